@@ -802,7 +802,7 @@ __global__ void __launch_bounds__(256) conv2d_wgrad_mfma(const WgradParams p) {
 
 // Weight gradient with both operand tiles loaded straight from global memory
 // into LDS (buffer loads with the LDS as destination), the forward direct
-// GEMM's pipeline (gemm.hip, gemm_f32_direct): BM x 64 tiles (BM = 128 or
+// GEMM's pipeline (gemm.hip, gemm_f32_direct_kg): BM x 64 tiles (BM = 128 or
 // 64), k-tiles of 16 pixels, 4 waves of (BM/2) x 32, two separate LDS
 // buffers and the k loop unrolled by two.  Both operands run along the
 // pixel index, so both live m-major, 64 bytes per row, chunk c (4 pixels)

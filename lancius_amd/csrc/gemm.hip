@@ -19,26 +19,10 @@
 #include <algorithm>
 #include <mutex>
 
-#include "common.hpp"
-#include "kernels.hpp"
+#include "gemm.hpp"
 
 namespace lancius {
 namespace {
-
-struct GemmParams {
-    float* C[LANCIUS_HIP_MAX_GROUP];
-    const float* A[LANCIUS_HIP_MAX_GROUP];
-    const float* R[LANCIUS_HIP_MAX_GROUP];     // residuals (may be null)
-    const float* B[LANCIUS_HIP_MAX_GROUP];
-    const float* bias[LANCIUS_HIP_MAX_GROUP];  // may be null
-    int M, N, K;
-    int act;
-    uint32_t tiles_m, tiles_n;
-    float* ws;   // split-K partials [count][splits][M][N]
-    unsigned* counters;  // fused skinny split-K: one arrival counter per (group, column block), zero between launches
-    int splits;  // K ranges (blockIdx.y), 1 = no split
-    int kchunk;  // K per split, a multiple of the k-tile
-};
 
 constexpr int kThreads = 256;
 
@@ -437,7 +421,7 @@ __global__ void __launch_bounds__(kThreads * KG, OCC) gemm_f32_mfma(const GemmPa
         }
         return;
     }
-    // (the activation chosen once per launch, as in gemm_f32_direct)
+    // (the activation chosen once per launch)
     const float* __restrict__ bias = p.bias[g];
     with_act(p.act, [&](auto act_c) {
         constexpr int ACT = decltype(act_c)::value;
@@ -463,236 +447,29 @@ __global__ void __launch_bounds__(kThreads * KG, OCC) gemm_f32_mfma(const GemmPa
     });
 }
 
-// 128x128 tiles, k-tiles of 16, 4 waves of 64x64, with both operand tiles
-// loaded straight from global memory into LDS (16-byte buffer loads with the
-// LDS as destination, gfx950): no register staging and no LDS store
-// instructions, and the next k-tile's loads have a whole k-tile of MFMAs to
-// land before the barrier that precedes their first read.  The two LDS
-// buffers are separate arrays and the loop is unrolled by two, so every
-// access names its buffer statically.
+// 64 x 64 tiles with both operand tiles loaded straight from global memory
+// into LDS (16-byte buffer loads with the LDS as destination, gfx950): no
+// register staging and no LDS store instructions, and the next k-tile's loads
+// have a whole k-tile of MFMAs to land before the barrier that precedes their
+// first read.
 //  * A (rows m0.., float4 chunks c of 4 k) lives m-major, 64 bytes per row;
 //    chunk c of row r sits at chunk c ^ ((r >> 2) & 3), so the 16-byte
 //    operand reads of 16 consecutive rows hit 16 different bank groups.
-//  * B (rows k, columns n0..) lives k-major, 512 bytes per row; chunk c of
-//    row k sits at chunk c ^ (8 * ((k >> 3) & 1)): the two lane halves, which
-//    read rows 8 apart, land on disjoint banks.
+//  * B (rows k, columns n0..) lives k-major; chunk c of row k sits at chunk
+//    c ^ (8 * ((k >> 3) & 1)): the two lane halves, which read rows 8 apart,
+//    land on disjoint banks.
 //  * Elements past K are zero because their loads use an offset past the
 //    buffer's end (which returns 0); rows past M and columns past N read the
 //    last row / column and only reach entries of C that are never stored.
 // Requires A, B non-transposed and float4-aligned (K, N multiples of 4) and
-// both operands under 2 GiB.  A and B use the same k pairing as the AMK
-// path: lane half h of the MFMAs takes k in [8h, 8h + 8).
-template <int OCC>
-__global__ void __launch_bounds__(256, OCC) gemm_f32_direct(const GemmParams p) {
-    constexpr int BM = 128, BN = 128, BK = 16;
-    constexpr int WM = 64, WN = 64, TM = 2, TN = 2;
-    typedef __attribute__((address_space(3))) void lds_void;
-    __shared__ __attribute__((aligned(16))) float As0[BM * BK];
-    __shared__ __attribute__((aligned(16))) float As1[BM * BK];
-    __shared__ __attribute__((aligned(16))) float Bs0[BK * BN];
-    __shared__ __attribute__((aligned(16))) float Bs1[BK * BN];
-
-    const int g = blockIdx.z;
-    const float* __restrict__ A = p.A[g];
-    const float* __restrict__ B = p.B[g];
-    float* __restrict__ C = p.C[g];
-    const float* __restrict__ R = p.R[g];
-    const int M = p.M, N = p.N, K = p.K;
-    const uint32_t ntiles = p.tiles_m * p.tiles_n;
-    uint32_t tm_id, tn_id;
-    grouped_tile(xcd_contiguous_id(blockIdx.x, ntiles), p.tiles_m, p.tiles_n, 4, tm_id, tn_id);
-    const int m0 = (int)tm_id * BM;
-    const int n0 = (int)tn_id * BN;
-
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 31, lk = lane >> 5;
-
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(A), 0, (int)((size_t)M * K * sizeof(float)), kBufferRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(B), 0, (int)((size_t)K * N * sizeof(float)), kBufferRsrcWord3);
-    constexpr int kOut = 0x7ffffff0;  // an offset past the end of any operand: the load returns 0
-
-    // This lane's two chunks of each tile (instruction i of wave w fills LDS
-    // chunks (2w + i) * 64 + lane).  Byte offsets at k0 = 0; per k-tile A
-    // moves 64 bytes and B 16 rows.
-    int a_row[2], a_k[2], b_kr[2];
-    int a_off0[2], b_off0[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int q = (2 * wave + i) * 64 + lane;
-        const int row = q >> 2, c = (q & 3) ^ ((row >> 2) & 3);
-        a_row[i] = row;
-        a_k[i] = 4 * c;
-        a_off0[i] = (min(m0 + row, M - 1) * K + 4 * c) * (int)sizeof(float);
-        const int kr = q >> 5, lc = (q & 31) ^ (((kr >> 3) & 1) << 3);
-        b_kr[i] = kr;
-        b_off0[i] = (kr * N + min(n0 + 4 * lc, N - 4)) * (int)sizeof(float);
-    }
-    auto load_tile = [&](float* As, float* Bs, int kt) {
-        const int k0 = kt * BK;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int ao = k0 + a_k[i] < K ? a_off0[i] + k0 * (int)sizeof(float) : kOut;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(As + (2 * wave + i) * 256), 16, ao, 0, 0, 0);
-            const int bo = k0 + b_kr[i] < K ? b_off0[i] + k0 * N * (int)sizeof(float) : kOut;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void*)(Bs + (2 * wave + i) * 256), 16, bo, 0, 0, 0);
-        }
-        // (compute places them between its first MFMAs)
-    };
-
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    // operand addresses (floats) of this lane, fixed over the k loop
-    int a_rd[TM][2];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int row = wm * WM + i * 32 + lr, c = 2 * lk + h;
-            a_rd[i][h] = row * BK + 4 * (c ^ ((row >> 2) & 3));
-        }
-    int b_rd[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int n = wn * WN + j * 32 + lr;
-        b_rd[j] = 8 * lk * BN + 4 * ((n >> 2) ^ (lk << 3)) + (n & 3);
-    }
-    auto compute = [&](const float* As, const float* Bs) {
-        f32x4 av[TM][2];
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) av[i][h] = *(const f32x4*)(As + a_rd[i][h]);
-#pragma unroll
-        for (int kp = 0; kp < 8; ++kp) {
-            float bf[TN];
-#pragma unroll
-            for (int j = 0; j < TN; ++j) bf[j] = Bs[b_rd[j] + kp * BN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][kp / 4][kp % 4], bf[j], acc[i][j], 0, 0, 0);
-        }
-        // the k-tile's four loads one after each of the first four MFMAs
-        // (the scheduler would otherwise sink them to the wait before the
-        // barrier)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // global load
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, TM * TN * 8 - 4, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    // k-tiles in pairs; when their count is odd the last pair's second tile
-    // lies wholly past K, loads as zeros and adds nothing.
-    const int pairs = (K + 2 * BK - 1) / (2 * BK);
-    load_tile(As0, Bs0, 0);
-    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-    __syncthreads();
-    for (int pr = 0; pr < pairs; ++pr) {
-        load_tile(As1, Bs1, 2 * pr + 1);
-        compute(As0, Bs0);
-        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-        __syncthreads();
-        // (unconditional, so the loads share the MFMAs' block: past K they
-        // read zeros, and the wait below covers them)
-        load_tile(As0, Bs0, 2 * pr + 2);
-        compute(As1, Bs1);
-        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-        __syncthreads();
-    }
-
-    // ---- epilogue: bias, activation, residual, one store -----------------
-    // The activation is chosen once per launch and a tile wholly inside C
-    // takes a copy without bounds checks: per element, a four-way switch
-    // and the row check made the unrolled epilogue thousands of branchy
-    // instructions, fetched by every CU at once at the end of the launch.
-    const float* __restrict__ bias = p.bias[g];
-    const int cb = n0 + wn * WN + lr;
-    float bv[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bv[j] = bias && cb + 32 * j < N ? bias[cb + 32 * j] : 0.0f;
-    const bool full = m0 + BM <= M && n0 + BN <= N;
-    with_act(p.act, [&](auto act_c) {
-        constexpr int ACT = decltype(act_c)::value;
-        if (full) {
-            // one 32 x 32 block at a time (a scheduling barrier between
-            // blocks keeps the residual loads from all being hoisted at once)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int i = 0; i < TM; ++i) {
-                    const size_t o0 = (size_t)(m0 + wm * WM + i * 32 + 4 * lk) * N + cb + 32 * j;
-                    float* __restrict__ cp = C + o0;
-                    if (R) {
-                        const float* __restrict__ rp = R + o0;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const size_t ro = (size_t)(8 * (r >> 2) + (r & 3)) * N;
-                            cp[ro] = act_fixed<ACT>(acc[i][j][r] + bv[j]) + rp[ro];
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            cp[(size_t)(8 * (r >> 2) + (r & 3)) * N] = act_fixed<ACT>(acc[i][j][r] + bv[j]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            return;
-        }
-        // a tile on the edge of C: the same blocks with bounds, the block's
-        // residual values loaded before its stores
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int col = cb + 32 * j;
-            if (col >= N) continue;
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const int rbase = m0 + wm * WM + i * 32 + 4 * lk;
-                float rv[16];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = rbase + 8 * (r >> 2) + (r & 3);
-                    rv[r] = R && row < M ? R[(size_t)row * N + col] : 0.0f;
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = rbase + 8 * (r >> 2) + (r & 3);
-                    if (row < M) {
-                        const float v = act_fixed<ACT>(acc[i][j][r] + bv[j]);
-                        C[(size_t)row * N + col] = R ? v + rv[r] : v;
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    });
-}
-
-// The direct-load pipeline of gemm_f32_direct for grids too small to give
-// every CU several tiles: BM x BM tiles (BM = 128, or 64 for the smallest
-// products) and KG k-groups of 4 waves in one workgroup.  Group g takes
-// k-tiles g, g + KG, g + 2 KG, ... with its own pair of LDS buffers (same
-// layouts and swizzles as gemm_f32_direct, scaled to BM), so a CU runs 4 KG
-// waves on its tile instead of 4.  At the end the groups' sums are added
-// through LDS in the fixed order (g0 + g1) + (g2 + g3), every wave taking a
-// share of the tile's epilogue: results are run-to-run identical.
-template <int BM, int KG, int BK = 16>
+// both operands under 2 GiB.  KG k-groups of 4 waves in one workgroup: group g
+// takes k-tiles g, g + KG, g + 2 KG, ... with its own pair of LDS buffers, so
+// a CU runs 4 KG waves on its tile instead of 4.  At the end the groups' sums
+// are added through LDS in the fixed order (g0 + g1) + (g2 + g3), every wave
+// taking a share of the tile's epilogue: results are run-to-run identical.
+template <int KG>
 __global__ void __launch_bounds__(256 * KG, 1) gemm_f32_direct_kg(const GemmParams p) {
-    constexpr int BN = BM;
-    static_assert(BK == 16 || BK == 32, "k-tile");
+    constexpr int BM = 64, BN = 64, BK = 16;
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
     constexpr int AI = BM * BK / 1024, BI = BN * BK / 1024;  // 16-byte loads per wave per k-tile
     constexpr int ACH = BK / 4;                                // 16-byte chunks of an A row
@@ -734,11 +511,10 @@ __global__ void __launch_bounds__(256 * KG, 1) gemm_f32_direct_kg(const GemmPara
     // A chunks: instruction i of wave gw fills chunks (AI gw + i) * 64 + lane
     // (row q / ACH, chunk (q % ACH) ^ aswz(row)); B chunks likewise (row
     // q / (BN / 4), chunk swizzled by 8 for the rows the second lane half
-    // reads).  With BK = 16 a row is 4 chunks (4 rows per 256 bytes of
-    // banks) and aswz(r) = (r >> 2) & 3; with BK = 32 it is 8 chunks (2 rows
-    // per 256 bytes) and aswz(r) = (r >> 1) & 7: either way the 16-byte
-    // reads of 16 consecutive rows at one chunk hit 16 different bank groups.
-    auto aswz = [](int row) { return BK == 16 ? (row >> 2) & 3 : (row >> 1) & 7; };
+    // reads).  A row is 4 chunks (4 rows per 256 bytes of banks): with
+    // aswz(r) = (r >> 2) & 3 the 16-byte reads of 16 consecutive rows at one
+    // chunk hit 16 different bank groups.
+    auto aswz = [](int row) { return (row >> 2) & 3; };
     constexpr int BHALF = BK / 2;  // B row of the second lane half's first k
     int a_k[AI], a_off0[AI], b_kr[BI], b_off0[BI];
 #pragma unroll
@@ -1203,6 +979,13 @@ __global__ void __launch_bounds__(256) splitk_reduce(const GemmParams p, int cou
     }
 }
 
+int launch_splitk_reduce(lancius_hip_ctx* ctx, const GemmParams& p, int count) {
+    const size_t total = (size_t)count * p.M * p.N;
+    const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 4096);
+    hipLaunchKernelGGL(splitk_reduce, dim3(blocks), dim3(256), 0, ctx->stream, p, count);
+    return check_launch("splitk_reduce");
+}
+
 // SPLITS: the configuration can be chosen for a split K (grids under 256
 // tiles); VECS: with float4 operand loads (false where the dispatch sends
 // every float4-shaped case of the configuration to a direct kernel).  Only
@@ -1244,20 +1027,14 @@ int launch_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec) {
                        ctx->stream, p);
 launched:
     if (int rc = check_launch("gemm_f32_mfma")) return rc;
-    if (split) {
-        const size_t total = (size_t)count * p.M * p.N;
-        const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 4096);
-        hipLaunchKernelGGL(splitk_reduce, dim3(blocks), dim3(256), 0, ctx->stream, p, count);
-        if (int rc = check_launch("splitk_reduce")) return rc;
-    }
-    return 0;
+    return split ? launch_splitk_reduce(ctx, p, count) : 0;
 }
 
 // Transposed operands are built for the two default tile shapes only.
 // Configurations 6 and 8 run grids of at least 256 tiles, which never split
-// K; with plain operands, configuration 6's float4 case is the direct
-// kernel's (the dispatch sends operands beyond its 2 GiB offsets to the
-// scalar variant).
+// K; with plain operands, configuration 6 (at least 768 tiles) is left with
+// operands beyond the split-product kernels' 32-bit offsets, and is built
+// with scalar loads only.
 template <bool TA, bool TB>
 int launch_by_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec, int cfg) {
     if constexpr (TA || TB) {
@@ -1406,6 +1183,65 @@ int arrival_counters(lancius_hip_ctx* ctx, const SplitStore* st, size_t n, unsig
 constexpr int kBK = 16;
 constexpr size_t kMaxSplitBytes = (size_t)256 << 20;
 
+// Which kernel a product takes when it is too large for the skinny one, from
+// what each costs on this chip (us, one launch alone, 256 CUs):
+//  * split-product tiles (gemm_f32_split): a round of one tile per CU costs a
+//    start and a time per unit of K.  Measured at 4096 x 4096 x K (256 x 256:
+//    one round) and 2048 x 2048 x 2048 (128 x 128: one round):
+//        256 x 256   11 + 0.137 K   (K = 512 84, 1024 157, 4096 584-600)
+//        256 x 128    9 + 0.074 K   (2048 x 1024 x 3072, 192 tiles: 70)
+//        128 x 128    7 + 0.041 K   (2048^3: 90, 448 x 64 x 128: 8.4)
+//    A round that fills only part of the chip runs at a higher clock: 0.6 +
+//    0.4 fill of the time per K (64 tiles of 256 x 256 at K = 2048: 209
+//    against 297).  Ranges of K over workgroups add the reduction launch and
+//    the partial sums' way through memory.
+//  * the fp32 kernels: 64 x 64 tiles run a round in 0.0155 K (1024^3 20.5),
+//    128 x 128 tiles in 0.065 K (2048^3 128, 1088 x 4608 x 3904 with B^T in
+//    two rounds 598), 64 x 64 tiles of transposed operands in 0.031 K;
+//    unaligned operands cost a third more (1537 x 1000 x 2999: 176); small
+//    grids take 5 + 0.03 K below K = 256 (448 x 64 x 128: 6.1) and split K
+//    over workgroups from there, at about 80 TFLOP/s of padded work plus 8 us
+//    (6936 x 7014 x 21: 176, 128 x 4096 x 4096: 51).
+struct GemmPlan {
+    int tile;       // kSplit* or -1: the fp32 kernels
+    size_t splits;  // kSplit128 only
+    double us;
+};
+
+GemmPlan gemm_plan(size_t count, size_t M, size_t K, size_t N, bool plain, bool vec) {
+    const double k = (double)K;
+    auto tiles = [&](size_t bm, size_t bn) { return count * ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    auto rounds = [](size_t t) { return (double)((t + 255) / 256); };
+    const size_t t64 = tiles(64, 64), t128 = tiles(128, 128);
+    double fp32;
+    if (t128 >= 256 && (!plain || !vec || K >= 2048))
+        fp32 = 4.0 + rounds(t128) * 0.065 * k;
+    else if (t64 >= (plain ? 192 : 256))
+        fp32 = 4.0 + (plain ? rounds(t64) * 0.0155 : (double)t64 / 256 * 0.031) * k;
+    else if (K < 256)
+        fp32 = 5.0 + 0.03 * k;
+    else
+        fp32 = 8.0 + (plain && K >= 2048 && t128 >= 16 ? (double)t128 * 128 * 128 : (double)t64 * 64 * 64) * 2e-6 * k / 80;
+    if (plain && !vec) fp32 *= 1.3;
+    const double out_bytes = 4.0 * (double)count * M * N;
+    fp32 += out_bytes / 6e6;
+    GemmPlan best{-1, 1, fp32};
+    if (t128 >= 768) best.us = 1e30;  // split products are ahead there down to K = 16 (4096 x 48 x 4096: 27 -> 18)
+    auto offer = [&](int tile, size_t splits, size_t t, double start, double per_k, double after) {
+        const double full = (double)(t / 256), fill = (double)(t % 256) / 256;
+        const double us = rounds(t) * start + (full + (fill > 0 ? 0.6 + 0.4 * fill : 0.0)) * per_k * k / (double)splits;
+        if (us + after < best.us) best = {tile, splits, us + after};
+    };
+    // (the one-sum tiles only where the fp32 kernels sum K in one chain too:
+    // smaller plain grids add two or four partial sums, which is more exact)
+    if (t128 >= 768 || !plain) offer(kSplit256, 1, tiles(256, 256), 11.0, 0.137, 0.0);
+    offer(kSplit256x128, 1, tiles(256, 128), 9.0, 0.074, 0.0);
+    offer(kSplit128, 1, t128, 7.0, 0.041, 0.0);
+    for (size_t s = 2; s <= 16 && K / s >= 256 && out_bytes * s <= (double)kScratchPartialBytes; ++s)
+        offer(kSplit128, s, t128 * s, 7.0, 0.041, 5.0 + out_bytes * (double)(s + 1) / 4e6);
+    return best;
+}
+
 // fixed: when not null, split-K partials and arrival counters go to its
 // buffers instead of the context's, and nothing is allocated.
 int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const float* const* A,
@@ -1494,20 +1330,44 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
         }
     }
 
+    const size_t big_tiles = count * ((M + 127) / 128) * ((N + 127) / 128);
+    // Products large enough for the bf16 matrix cores' split products
+    // (gemm_split.hip); both operands transposed, or one beyond 32-bit
+    // offsets, stay with the fp32 kernels.
+    const bool split_fits = (M + 96) * (K + 96) * sizeof(float) < kSplitMaxBytes &&
+                            (K + 96) * (N + 96) * sizeof(float) < kSplitMaxBytes &&
+                            (M + 256) * (N + 256) * sizeof(float) < kSplitMaxBytes;
+    if (!(ta && tb) && split_fits && (K >= 32 || big_tiles >= 768)) {
+        const GemmPlan plan = gemm_plan(count, M, K, N, !ta && !tb, vec);
+        if (plan.tile >= 0) {
+            const size_t steps = (K + 31) / 32, chunk = (steps + plan.splits - 1) / plan.splits;
+            p.splits = (int)((steps + chunk - 1) / chunk);  // no empty K range
+            p.kchunk = (int)(chunk * 32);
+            if (p.splits > 1) {
+                void* ws = nullptr;
+                if (int rc = partials(ctx, fixed, count * p.splits * M * N * sizeof(float), &ws)) return rc;
+                p.ws = (float*)ws;
+            }
+            if (int rc = launch_gemm_split(ctx, p, (int)count, ta, tb, plan.tile)) return rc;
+            if (p.splits > 1)
+                if (int rc = launch_splitk_reduce(ctx, p, (int)count)) return rc;
+            return ok();
+        }
+    }
+
     // Configurations (BM x BN / BK, k-groups): 2 = 64x64/16, 6 = 128x128/16
     // built for 4 workgroups per CU, 7 = 128x128/32 x2, 8 = 128x128/32 x4,
     // 9 = 64x64/64 x4.  Chosen by the number of 128x128 tiles (one per CU
     // fills the chip once), measured on MI355X:
-    //  * >= 768: 6 (4096^3: 112 TFLOP/s);
+    //  * >= 768: 6 (operands beyond 32-bit offsets);
     //  * 384 .. 767: 7 (two 8-wave workgroups per CU);
-    //  * 256 .. 383: 8, 16 waves on the CU's one tile (2048^3: 205 -> 190
-    //    us; 4096x1024x1024: 110 -> 103 us);
+    //  * 256 .. 383: 8, 16 waves on the CU's one tile (4096x1024x1024: 110 ->
+    //    103 us);
     //  * fewer, K >= 2048: 7 with split-K (1024x4096x1024: 137 -> 103 us);
     //  * fewer, shorter K: 9 (1024^3: 38.9 -> 34.0 us), or 2 for small
     //    grids and transposed operands.
     // Split-K when the grid still leaves CUs idle and K is long enough:
     // enough K ranges for ~512 workgroups, each >= 128 deep.
-    const size_t big_tiles = count * ((M + 127) / 128) * ((N + 127) / 128);
     const size_t t64 = count * ((M + 63) / 64) * ((N + 63) / 64);
     const bool plain = !ta && !tb;
     int cfg;
@@ -1541,68 +1401,32 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
     }
     p.splits = (int)splits;
     p.kchunk = (int)(chunk_tiles * bk);
-    // 128x128 tiles loaded straight into LDS (gemm_f32_direct)
-    if (cfg == 6 && splits == 1 && vec && !ta && !tb &&
-        M * K * sizeof(float) < ((size_t)1 << 31) && K * N * sizeof(float) < ((size_t)1 << 31)) {
-        p.tiles_m = (uint32_t)((M + 127) / 128);
-        p.tiles_n = (uint32_t)((N + 127) / 128);
-        // the k-tile's four loads one after each of the first four MFMAs
-        // (measured 143.0 -> 144.4 TFLOP/s at 4096^3; a burst before the
-        // MFMAs, or one load per 2, 4 or 7 MFMAs, ran slower)
-        hipLaunchKernelGGL(gemm_f32_direct<4>, dim3(p.tiles_m * p.tiles_n, 1, (unsigned)count), dim3(256), 0, ctx->stream, p);
-        if (int rc = check_launch("gemm_f32_direct")) return rc;
-        return ok();
-    }
-    // Grids that give a CU about one 128 x 128 tile (or one 64 x 64 tile):
-    // the direct-load pipeline with the K loop spread over k-groups of
-    // 4 waves inside the workgroup (gemm_f32_direct_kg)
+    // Grids that give a CU a few 64 x 64 tiles: the direct-load pipeline with
+    // the K loop spread over k-groups of 4 waves inside the workgroup, 4 of
+    // them when that gives about one tile per CU and 2 otherwise
+    // (gemm_f32_direct_kg; against the staged kernels: 1024^3 27.0 -> 20.5 us,
+    // 4096x1024x1024 82.4 -> 69.3).  At least 192 tiles: with 128 to 191 the
+    // split-K tiled kernels below are faster (128x2048x4096 38.1 -> 35.0 us,
+    // 256x2048x2048 36.2 -> 34.4; 192 tiles, 192x4096x4096, measured 71.7
+    // against 84.0 us split).  K-tiles of 32 (half the barriers per k)
+    // measured no better (1024^3 23.9 -> 24.3 us).
     if (vec && plain && M * K * sizeof(float) < ((size_t)1 << 31) && K * N * sizeof(float) < ((size_t)1 << 31) &&
-        K >= 256 && big_tiles < 768) {
-        // 64 x 64 tiles, with 4 k-groups when that gives about one tile per
-        // CU and 2 otherwise; 128 x 128 tiles with 4 k-groups (16 waves, 100
-        // registers each) for K >= 2048 with >= 192 of them.
-        // Measured on MI355X (old dispatch -> this): 1024^3 27.0 -> 23.7 us,
-        // 2048^3 146.0 -> 135.6, 4096x1024x1024 82.4 -> 71.3,
-        // 1024x4096x1024 84.4 -> 76.4, 4096x4096x1024 275.2 -> 257.3,
-        // 3000x1000x2000 145.8 -> 104.3.  The 128 x 128 tiles with 4 k-groups
-        // of 16-deep k-tiles against 2 k-groups of 32-deep ones (one box, the
-        // two builds alternated): 2048^3 131.3 -> 129.0 us, 2048x4096x2048
-        // 251.1 -> 246.7, 2048x2048x4096 259.3 -> 254.2, four grouped
-        // 1024x4096x1024 (bias and residual) 259.8 -> 251.4.  At K = 1024 they
-        // lose to 64 x 64 tiles unless the grid is exactly 256 of them (3072 x
-        // 1024 x 1024: 54.9 -> 69.2 us; 4096 x 1024 x 1024: 70.5 -> 69.9).
-        // (128 x 128 tiles from 256 of them: with 192 to 255 the 64 x 64
-        // tiles measured faster, 768x4096x4096 245.5 -> 195.5 us and
-        // 4096x2048x768 127.7 -> 101.8 us, one box, builds alternated)
-        const int bm_kg = K >= 2048 && big_tiles >= 256 ? 128 : 64;
-        const int kg = bm_kg == 128 || t64 <= 384 ? 4 : 2;
-        const size_t kg_tiles = count * ((M + bm_kg - 1) / bm_kg) * ((N + bm_kg - 1) / bm_kg);
-        // at least 192 tiles: with 128 to 191 the split-K tiled kernels
-        // below are faster (128x4096x4096 72.0 -> 52.2 us, 4096x4096x128
-        // 74.6 -> 51.3 us, 96x4096x4096 71.5 -> 51.5 us, 128x2048x4096 38.1
-        // -> 35.0 us; 192 tiles, e.g. 192x4096x4096, measured 71.7 against
-        // 84.0 us split)
-        if (kg_tiles >= 192) {
-            p.tiles_m = (uint32_t)((M + bm_kg - 1) / bm_kg);
-            p.tiles_n = (uint32_t)((N + bm_kg - 1) / bm_kg);
-            // k-tiles of 16: with 32 (half the barriers per k) the 64 x 64
-            // tiles measured no better (1024^3 23.9 -> 24.3 us, four grouped
-            // 72.1 -> 72.7 us), and 128 x 128 tiles with 4 k-groups would
-            // need 256 KB of LDS
-            void (*kern)(const GemmParams) = bm_kg == 128 ? gemm_f32_direct_kg<128, 4>
-                                                          : (kg == 2 ? gemm_f32_direct_kg<64, 2> : gemm_f32_direct_kg<64, 4>);
-            hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n, 1, (unsigned)count), dim3(256 * kg), 0,
-                               ctx->stream, p);
-            if (int rc = check_launch("gemm_f32_direct_kg")) return rc;
-            return ok();
-        }
+        K >= 256 && big_tiles < 768 && t64 >= 192) {
+        p.tiles_m = (uint32_t)((M + 63) / 64);
+        p.tiles_n = (uint32_t)((N + 63) / 64);
+        const int kg = t64 <= 384 ? 4 : 2;
+        hipLaunchKernelGGL((kg == 2 ? gemm_f32_direct_kg<2> : gemm_f32_direct_kg<4>),
+                           dim3(p.tiles_m * p.tiles_n, 1, (unsigned)count), dim3(256 * kg), 0, ctx->stream, p);
+        if (int rc = check_launch("gemm_f32_direct_kg")) return rc;
+        return ok();
     }
     if (splits > 1) {
         void* ws = nullptr;
         if (int rc = partials(ctx, fixed, count * splits * M * N * sizeof(float), &ws)) return rc;
         p.ws = (float*)ws;
     }
-    // plain configuration-6 operands beyond the direct kernel's offsets: scalar loads
+    // plain configuration-6 grids come here only with operands beyond 32-bit
+    // offsets: scalar loads
     if (cfg == 6 && plain) vec = false;
     int rc;
     if (ta && tb)

@@ -1,0 +1,73 @@
+// fp32 products on the bf16 matrix cores, without giving up fp32 accuracy.
+//
+// An fp32 value is the exact sum of three bf16 values: h = bf16(x),
+// m = bf16(x - h), l = bf16(x - h - m) (round to nearest; the two
+// differences are exact in fp32, and 3 x 8 significand bits cover its 24).
+// A product x y is then formed from six bf16 products,
+//     hh' + (hm' + mh') + (mm' + hl' + lh'),
+// each exact in the fp32 accumulator's input.  The three products left out
+// (ml', lm', ll') are below 2^-26 of x y, under half an fp32 ulp.  The
+// accumulator is fp32 as before, and the six are summed from the smallest
+// terms up.  v_mfma_f32_32x32x16_bf16 does 16 times the multiply-adds per
+// cycle of v_mfma_f32_32x32x2_f32, so six of them leave a factor of 2.7 in
+// matrix-core cycles.
+//
+// Range: bf16 has fp32's exponents, so nothing overflows or vanishes except
+// at the ends: x above the largest bf16 rounds to infinity, and infinities
+// and NaN give NaN in the differences.  Every such case makes the affected
+// sums non-finite, and the kernels recompute a tile whose sums are not all
+// finite with the fp32 matrix instructions, so those inputs give what they
+// give in fp32.  Below 2^-110 the low parts reach bf16's subnormals (which
+// the matrix cores keep) and end at 2^-133.
+#pragma once
+
+#include "kernels.hpp"
+
+namespace lancius {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+// One lane's MFMA operand: eight consecutive k of one row, in three parts.
+struct SplitOperand {
+    bf16x8 h, m, l;
+};
+
+// bf16 of two floats in one register, and those two back as floats.
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
+
+__device__ __forceinline__ SplitOperand split8(f32x8 x) {
+    u32x4 h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = x[2 * i], b = x[2 * i + 1];
+        h[i] = pack_bf16(a, b);
+        a -= __builtin_bit_cast(float, h[i] << 16);
+        b -= __builtin_bit_cast(float, h[i] & 0xffff0000u);
+        m[i] = pack_bf16(a, b);
+        a -= __builtin_bit_cast(float, m[i] << 16);
+        b -= __builtin_bit_cast(float, m[i] & 0xffff0000u);
+        l[i] = pack_bf16(a, b);
+    }
+    return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+
+__device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// c + a . b over 16 k, smallest terms first.
+__device__ __forceinline__ f32x16 mfma_split(const SplitOperand& a, const SplitOperand& b, f32x16 c) {
+    c = mfma_bf16(a.l, b.h, c);
+    c = mfma_bf16(a.h, b.l, c);
+    c = mfma_bf16(a.m, b.m, c);
+    c = mfma_bf16(a.m, b.h, c);
+    c = mfma_bf16(a.h, b.m, c);
+    return mfma_bf16(a.h, b.h, c);
+}
+
+}  // namespace lancius
