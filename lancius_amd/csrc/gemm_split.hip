@@ -231,7 +231,9 @@ __global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, 2) gemm_f32_s
         k_loop(std::integral_constant<bool, true>{});
     else
         k_loop(std::integral_constant<bool, false>{});
+    settle(acc);
     if constexpr (MODE == kTwoSums) {
+        settle(low);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -289,6 +291,7 @@ __global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, 2) gemm_f32_s
                     const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, bo, 0, 0));
                     s = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, s, 0, 0, 0);
                 }
+                settle(s);
                 acc[i][j] = s;
             }
     }

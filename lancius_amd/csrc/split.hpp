@@ -70,4 +70,32 @@ __device__ __forceinline__ f32x16 mfma_split(const SplitOperand& a, const SplitO
     return mfma_bf16(a.h, b.h, c);
 }
 
+// An instruction that reads a matrix instruction's result needs wait states
+// that the compiler counts; across a branch it has been seen to count them
+// along the longer of two paths only (the reader got registers 14 and 15 of a
+// 32 x 32 result from before the last product).  So a result that is read
+// behind control flow passes one of these first.
+//  settle: the value is complete here, whatever follows (20 wait states).
+//  pin: the instruction that computed the value stays in this block, where
+//  the count is right; for values that vector instructions have already read
+//  out of the matrix result.
+__device__ __forceinline__ void pin(f32x16& c) { asm volatile("" : "+v"(c)); }
+template <int M, int N>
+__device__ __forceinline__ void settle(f32x16 (&c)[M][N]) {
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < N; ++j) pin(c[i][j]);
+    asm volatile("s_nop 15\n\ts_nop 3");
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < N; ++j) pin(c[i][j]);
+}
+__device__ __forceinline__ void settle(f32x16& c) {
+    pin(c);
+    asm volatile("s_nop 15\n\ts_nop 3");
+    pin(c);
+}
+
 }  // namespace lancius
