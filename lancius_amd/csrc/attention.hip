@@ -25,34 +25,12 @@
 
 #include <algorithm>
 
-#include "common.hpp"
-#include "kernels.hpp"
+#include "attention.hpp"
 
 namespace lancius {
 namespace {
 
-struct AttnParams {
-    float* O[LANCIUS_HIP_MAX_GROUP];
-    const float* Q[LANCIUS_HIP_MAX_GROUP];
-    const float* K[LANCIUS_HIP_MAX_GROUP];
-    const float* V[LANCIUS_HIP_MAX_GROUP];
-    int batch;  // batches per group entry
-    int S, H, D;   // queries per sequence, query heads, head dim
-    int Skv, Hkv;  // keys per sequence, K/V heads (query head h reads K/V head h / (H / Hkv))
-    int causal;    // query i sees keys j <= i + (Skv - S)
-    float qscale;  // scale * log2(e)
-    int q_tiles;
-    int pair_tiles;  // causal grid small enough to be resident at once (see attention_mfma)
-    int Z;         // count * batch independent problems
-};
-
 constexpr int kBQ = 128;   // queries per workgroup (32 per wave)
-
-// 2^x as the one v_exp_f32.  exp2f adds a range fix-up (compare, select,
-// add, select, ldexp: five more instructions) that only changes results
-// below 2^-126; the softmax exponents here are <= 0 and a probability under
-// 2^-126 does not move a sum that is >= 1.
-__device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // D = head dim (a multiple of 32, at most 128); BKV = keys per LDS block
 // (64 for D <= 64, 32 above, so the K/V blocks of two workgroups fit a
@@ -824,6 +802,22 @@ int attention_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* O, cons
     p.Z = (int)z;
     // the MFMA kernel addresses a sequence's K and V rows with 32-bit buffer offsets
     if (vec && D % 32 == 0 && D <= 128 && Skv * Hkv * D * sizeof(float) < ((size_t)1 << 31) - 64) {
+        const size_t cus = (size_t)cu_count(ctx);
+        const size_t qt64 = (S + 63) / 64, t64 = qt64 * H * z;
+        // The split-product kernel, except where one or two steps of keys do
+        // not pay for its start (up to 64 keys: B3 H16 D32 S=52 5.9 against
+        // 6.7 us, B2 H2 D96 S=64 11.0 against 12.1) and for D = 64 grids of at
+        // most one 64-query tile per CU (B1 H16 S=512 25.8 against 28.3 us,
+        // B2 H8 S=256 15.1 against 17.7; at 288 tiles, B6 H16 S=149
+        // non-causal, 18.8 against 15.6 the other way).  Elsewhere, fp32
+        // kernel -> split products: B8 H16 D64 S=2048 causal 555 -> 407 us,
+        // S=512 causal 47.3 -> 39.5, B4 S=1024 causal 81.3 -> 67.9; D128 B8
+        // S=2048 2102 -> 1449, B4 q1024 kv2048 H32/8 824 -> 548; D32 B8
+        // S=2048 causal 298 -> 222; D96 B2 H12 S=1024 causal 117 -> 68.
+        if (Skv > 64 && !(D == 64 && t64 <= cus) && (Skv + 128) * Hkv * D * sizeof(float) < ((size_t)1 << 31)) {
+            if (int rc = launch_attention_split(ctx, p)) return rc;
+            return ok();
+        }
         // D = 64 grids of at most three 64-query tiles per CU: 4-wave
         // workgroups with one LDS buffer, three resident per CU, where the
         // 128-query grid leaves CUs idle or half-loaded.  Measured against
@@ -837,8 +831,6 @@ int attention_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* O, cons
         // tiles per CU (B8 S=512, B4 S=1024) it does not fit (three
         // workgroups a CU by registers).
         {
-            const size_t cus = (size_t)cu_count(ctx);
-            const size_t qt64 = (S + 63) / 64, t64 = qt64 * H * z;
             const size_t t128 = (S + kBQ - 1) / kBQ * H * z;
             if (D == 64 && t64 <= 3 * cus && (causal || t128 % cus != 0)) {
                 p.q_tiles = (int)qt64;
