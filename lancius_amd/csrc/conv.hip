@@ -18,9 +18,9 @@
 // lanes 0..31 of a register cover 32 consecutive pixels of one channel.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 
-#include "common.hpp"
-#include "kernels.hpp"
+#include "conv.hpp"
 
 namespace lancius {
 namespace {
@@ -1143,6 +1143,53 @@ int default_tile(size_t C_out) { return C_out > 64 ? 1 : C_out > 32 ? 2 : 3; }
 template <int KH_T, int KW_T>
 int launch_tile(lancius_hip_ctx* ctx, ConvParams& p, int tile);
 
+// What the two kernels take for a convolution, in us, fitted to both over 140
+// shapes (one box; K = C_in KH KW, M = C_out, one tile alone per CU unless
+// said).  Split products: 128 x 128 tiles 8 + 0.034 K (N1 256->512 14^2 84,
+// N6 208->240 5x5 38x16 186), two a CU past 256 tiles 9 + 0.0675 K a round of
+// 512 (N32 64->128 56^2 99); 64 x 128 tiles 8 + 0.0235 K, 0.06 K a round of 512
+// (N32 128->64 56^2 123).
+double conv_split_us(const ConvSplitParams& sp) {
+    const double k = (double)sp.KH * sp.KW * sp.C16, t = (double)conv_split_tiles(sp);
+    const bool wide = sp.C_out > 64;
+    if (t <= 256) return 8.0 + (wide ? 0.034 : 0.0235) * k;
+    return 9.0 * std::max(1.0, t / 512) + (wide ? 0.0675 : 0.06) * k * std::max(0.8, t / 512);
+}
+// fp32: conv2d_direct's 128 x 64 (64 x 64) tiles 0.0365 K (0.0196 K) a round of
+// 256; under half the CUs K is shared by up to 8 workgroups at 0.72 (0.42) us a
+// k-tile of 16 and 2.5 us more for each (N1 64->128 56^2 23.5, N1 256->512 14^2
+// 40); the 32 x 128 implicit GEMM 0.04 K a round of 384, and channel counts that are no
+// multiple of 16 (4) 0.085 K (N1 53->153 42x38 47, N24 12->20 5x5 41x92 71).
+double conv_fp32_us(const ConvParams& q) {
+    const double k = (double)q.Kdim, P = (double)q.Ptotal;
+    const bool aligned = q.C_in % 16 == 0 && q.C_out % 4 == 0;
+    const double rows = q.C_out > 64 ? std::ceil(q.C_out / 128.0) : std::ceil(q.C_out / 64.0);
+    if (!aligned || q.C_out <= 32) {
+        const double t = q.C_out <= 32 ? std::ceil(P / 128) : rows * std::ceil(P / 64);
+        return 5.0 + (aligned ? 0.04 : 0.085) * k * std::max(1.0, t / (aligned ? 384 : 256));
+    }
+    const double t = rows * std::ceil(P / 64), kt = k / 16;
+    const bool wide = q.C_out > 64;
+    if (t >= 256) return 6.0 + (wide ? 0.0365 : 0.0196) * k * t / 256;
+    const double ways = t < 128 ? std::min(std::min(8.0, 256 / t), std::max(1.0, std::floor(kt / 18))) : 1.0;
+    return 4.5 + (wide ? 0.72 : 0.42) * kt / ways + 2.5 * (ways - 1);
+}
+
+// The convolution q as split products (conv_split.hip), where they are the
+// faster kernel (by the estimates, with a tenth to spare).
+bool use_split(const ConvParams& q, ConvSplitParams* sp) {
+    *sp = ConvSplitParams{q.out, q.in, q.wt, q.bias, q.N, q.C_in, (q.C_in + 15) / 16 * 16, q.H, q.W, q.C_out, q.KH, q.KW,
+                          q.stride, q.pad, q.Ho, q.Wo, 0, q.act, 0};
+    if (q.prep == 2) {  // the gradient of a convolution of stride 1
+        sp->dgrad = 1;
+        sp->pad = q.KH - 1 - q.pad;
+    }
+    if (!conv_split_fits(*sp)) return false;
+    // (a ragged channel count has the filter laid out for the call, 4 us)
+    const double prep = q.prep == 1 && (q.C_in % 16 != 0 || q.C_out % 4 != 0) ? 4.0 : 0.0;
+    return (conv_split_us(*sp) + prep) * 1.1 < conv_fp32_us(q);
+}
+
 // One launch per run of images whose input stays under 2 GiB (the direct
 // kernel's 32-bit input offsets); the images of a conv are independent, so
 // the split changes no result.  p describes the whole batch.
@@ -1156,6 +1203,11 @@ int launch_batches(lancius_hip_ctx* ctx, const ConvParams& p, int tile) {
         q.in = p.in + n0 * img_in;
         q.out = p.out + n0 * img_out;
         q.Ptotal = (long long)q.N * p.Ho * p.Wo;
+        ConvSplitParams sp{};
+        if (use_split(q, &sp)) {
+            if (int rc = launch_conv_split(ctx, sp, p.prep == 0 ? nullptr : p.prep == 2 ? p.w_src : p.w)) return rc;
+            continue;
+        }
         const int rc = (p.KH == 3 && p.KW == 3) ? launch_tile<3, 3>(ctx, q, tile) : launch_tile<0, 0>(ctx, q, tile);
         if (rc) return rc;
     }
@@ -1282,6 +1334,16 @@ extern "C" int lancius_hip_conv2d_bwd_input_f32(lancius_hip_ctx* ctx, float* dx,
     const bool as_conv = stride == 1 && K_h == K_w && pad + 1 <= K_h && H_out > 0 && W_out > 0 &&
                          H + 2 * pad + 1 == H_out + K_h && W + 2 * pad + 1 == W_out + K_w;
     if (!as_conv) {
+        ConvSplitParams sp{dx, dy, nullptr, nullptr, (int)N, (int)C_out, (int)((C_out + 15) / 16 * 16), (int)H_out, (int)W_out,
+                           (int)C_in, (int)K_h, (int)K_w, (int)stride, (int)pad, (int)H, (int)W, 1, LANCIUS_HIP_ACT_NONE, 0};
+        // (up to a dozen products an element, or sizes beyond its offsets, the
+        // split-product kernel leaves to the direct one: N15 4->8 1x1 107x11
+        // 6.1 us against 8.6; N16 64->128 3x3 56^2 the other way, 3263
+        // against 32)
+        if (C_out * K_h * K_w > 12 && stride <= 16 && K_h < (1u << 15) && K_w < (1u << 15) && C_out > 0 && pad < (1u << 30) && conv_split_fits(sp)) {
+            const int rc = launch_conv_split(ctx, sp, w);
+            return rc ? rc : ok();
+        }
         const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>((total + 255) / 256, 16384));
         hipLaunchKernelGGL(dgrad_direct, dim3(grid), dim3(256), 0, ctx->stream, dx, dy, w, (int)N, (int)C_in, (int)H,
                            (int)W, (int)C_out, (int)H_out, (int)W_out, (int)K_h, (int)K_w, (int)stride, (int)pad);

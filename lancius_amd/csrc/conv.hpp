@@ -1,0 +1,30 @@
+// What the convolution translation units share.
+#pragma once
+
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace lancius {
+
+// The split-product convolution (conv_split.hip): out [N][C_out][Ho][Wo] from
+// in [N][C_in][H][W] and the filter matrix wt.  Forward: out of a KH x KW
+// convolution of `stride` and `pad`, wt [C_out][KH KW][C16].  dgrad: in = dy,
+// out = dx of such a convolution (the names follow this product: C_in is dy's
+// channels).  conv_split_fits says
+// whether the sizes stay within the kernel's 32-bit offsets.
+struct ConvSplitParams {
+    float* out;
+    const float* in;
+    const float* wt;
+    const float* bias;  // may be null
+    int N, C_in, C16, H, W, C_out, KH, KW, stride, pad, Ho, Wo;  // C16: C_in rounded up to 16
+    int dgrad, act;
+    uint32_t tiles_m;  // set by the launch
+};
+bool conv_split_fits(const ConvSplitParams& p);
+size_t conv_split_weight_bytes(const ConvSplitParams& p);
+size_t conv_split_tiles(const ConvSplitParams& p);  // workgroups of the launch
+// w: the filter [out][in][KH][KW] to lay out first (null: p.wt is ready).
+int launch_conv_split(lancius_hip_ctx* ctx, ConvSplitParams& p, const float* w);
+
+}  // namespace lancius

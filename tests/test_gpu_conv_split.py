@@ -1,0 +1,125 @@
+"""The split-product convolution (lancius_amd/csrc/conv_split.hip): channel,
+pixel and tap counts at the edges of its tiles, strides, the classes of strided
+input gradients, and non-finite inputs, against fp64."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import oracle
+from lancius_amd import ACT_NONE, ACT_RELU, prng
+from tests.conftest import case
+
+pytestmark = pytest.mark.gpu
+
+
+def _out(H, K, stride, pad):
+    return (H + 2 * pad - K) // stride + 1
+
+
+def _forward(dev, x, w, bias, stride, pad, act, packed):
+    N, C_in, H, W = x.shape
+    C_out, _, KH, KW = w.shape
+    Ho, Wo = _out(H, KH, stride, pad), _out(W, KW, stride, pad)
+    n = N * C_out * Ho * Wo
+    dx, dw, do = dev.upload(x), dev.upload(w), dev.alloc(4 * n + 4096)
+    db = dev.upload(bias) if bias is not None else None
+    dev.fill(do, 7.0, n + 1024)
+    if packed:
+        pk = dev.alloc(dev.conv2d_packed_bytes(C_out, C_in, KH, KW))
+        dev.conv2d_pack_weight(pk, dw, C_out, C_in, KH, KW)
+        dev.conv2d_packed(do, dx, pk, db, N, C_in, H, W, C_out, KH, KW, stride, pad, act)
+        pk.free()
+    else:
+        dev.conv2d(do, dx, dw, db, N, C_in, H, W, C_out, KH, KW, stride, pad, act)
+    got = dev.download(do, (n + 1024,))
+    assert (got[n:] == 7.0).all()  # nothing is stored past the output
+    for b in (dx, dw, do, db):
+        if b is not None:
+            b.free()
+    return got[:n].reshape(N, C_out, Ho, Wo)
+
+
+def _bwd_input(dev, dy, w, H, W, stride, pad):
+    N, C_out, Ho, Wo = dy.shape
+    _, C_in, KH, KW = w.shape
+    n = N * C_in * H * W
+    dg, dw, do = dev.upload(dy), dev.upload(w), dev.alloc(4 * n + 4096)
+    dev.fill(do, 7.0, n + 1024)
+    dev.conv2d_bwd_input(do, dg, dw, N, C_in, H, W, C_out, Ho, Wo, KH, KW, stride, pad)
+    got = dev.download(do, (n + 1024,))
+    assert (got[n:] == 7.0).all()
+    for b in (dg, dw, do):
+        b.free()
+    return got[:n].reshape(N, C_in, H, W)
+
+
+# (N, C_in, H, W, C_out, KH, KW, stride, pad, packed)
+FORWARD = [
+    (9, 64, 40, 36, 128, 3, 3, 1, 1, True),     # whole tiles, a tile a CU or less
+    (40, 32, 31, 33, 132, 3, 3, 1, 1, True),    # four channels past a tile, two tiles a CU
+    (3, 48, 57, 55, 96, 5, 5, 2, 2, True),      # stride 2, ragged pixels
+    (2, 37, 40, 41, 70, 3, 5, 1, 2, False),     # channels padded to 48, an oblong filter
+    (2, 96, 30, 30, 24, 7, 7, 3, 0, False),     # few output channels, stride 3, no padding
+    (1, 13, 64, 64, 51, 5, 5, 1, 2, False),
+]
+
+
+@pytest.mark.parametrize("N,C_in,H,W,C_out,KH,KW,stride,pad,packed", FORWARD)
+def test_conv_split_forward(dev, N, C_in, H, W, C_out, KH, KW, stride, pad, packed):
+    case(f"conv split forward {N} {C_in}->{C_out} {H}x{W} {KH}x{KW} stride {stride}")
+    x = prng.normal(6000, (N, C_in, H, W))
+    w = prng.normal(6001, (C_out, C_in, KH, KW), std=float(np.sqrt(2.0 / (C_in * KH * KW))))
+    b = prng.normal(6002, (C_out,))
+    act = ACT_RELU if stride == 1 else ACT_NONE
+    got = _forward(dev, x, w, b, stride, pad, act, packed)
+    ref = F.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), torch.from_numpy(b).double(), stride, pad)
+    ref = (F.relu(ref) if act == ACT_RELU else ref).numpy()
+    assert oracle.normwise_error(got, ref) <= oracle.tolerance(C_in * KH * KW)
+
+
+# (N, C_in, H, W, C_out, KH, KW, stride, pad)
+GRADIENT = [
+    (8, 64, 40, 36, 128, 3, 3, 1, 1),
+    (2, 96, 33, 31, 48, 5, 5, 1, 2),
+    (3, 40, 33, 30, 72, 3, 3, 2, 1),     # classes of different sizes
+    (2, 130, 20, 23, 37, 5, 5, 2, 2),    # dy's channels padded to 48
+    (2, 24, 32, 32, 48, 1, 1, 2, 0),     # three classes without a tap
+    (1, 20, 29, 31, 33, 7, 5, 3, 2),
+    (2, 16, 19, 40, 64, 3, 3, 4, 0),     # rows that no window reaches
+]
+
+
+@pytest.mark.parametrize("N,C_in,H,W,C_out,KH,KW,stride,pad", GRADIENT)
+def test_conv_split_bwd_input(dev, N, C_in, H, W, C_out, KH, KW, stride, pad):
+    case(f"conv split gradient {N} {C_in}->{C_out} {H}x{W} {KH}x{KW} stride {stride}")
+    Ho, Wo = _out(H, KH, stride, pad), _out(W, KW, stride, pad)
+    dy = prng.normal(6100, (N, C_out, Ho, Wo))
+    w = prng.normal(6101, (C_out, C_in, KH, KW), std=float(np.sqrt(2.0 / (C_out * KH * KW))))
+    got = _bwd_input(dev, dy, w, H, W, stride, pad)
+    x = torch.zeros(N, C_in, H, W, dtype=torch.float64, requires_grad=True)
+    F.conv2d(x, torch.from_numpy(w).double(), None, stride, pad).backward(torch.from_numpy(dy).double())
+    assert oracle.normwise_error(got, x.grad.numpy()) <= oracle.tolerance(C_out * KH * KW)
+
+
+@pytest.mark.parametrize("stride", [1, 2])
+def test_conv_split_non_finite(dev, stride):
+    """Infinities, NaN and values above the largest bf16 reach the outputs
+    whose windows hold them, with fp32's signs, and no others."""
+    N, C_in, H, W, C_out = 9, 64, 40, 36, 128
+    case(f"conv split non-finite stride {stride}")
+    x = prng.normal(6200, (N, C_in, H, W))
+    w = prng.normal(6201, (C_out, C_in, 3, 3), std=0.06)
+    x[0, 3, 5, 7], x[2, 60, 20, 20] = np.inf, np.nan
+    x[4, 10, 11, 12] = np.float32(3.4e38)  # rounds to infinity as bf16
+    w[7, 10] *= np.float32(2.0 ** -20)
+    got = _forward(dev, x, w, None, stride, 1, ACT_NONE, True)
+    ref = F.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), None, stride, 1).numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(got[inf], ref[inf].astype(np.float32))
+    big = np.isfinite(ref) & (np.abs(ref) > 1e20)
+    assert big.any()
+    for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
+        err = oracle.normwise_error(np.where(part, got, 0).astype(np.float64) * scale, np.where(part, ref, 0) * scale)
+        assert err <= oracle.tolerance(C_in * 9)
