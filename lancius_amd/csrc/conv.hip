@@ -1010,22 +1010,51 @@ __global__ void __launch_bounds__(256, 2) conv2d_wgrad_direct(const WgradParams 
 }
 
 // A workgroup per 64 consecutive weights: lane l of wave g adds splits g,
-// g+4, g+8, ... of weight l in order (a wave reads 256 contiguous bytes of a
-// split's partials), then wave 0 adds the four sums in wave order: a fixed
-// order, so results are identical from run to run.  (One wave per weight,
+// g+GROUPS, g+2 GROUPS, ... of weight l in order (a wave reads 256 contiguous
+// bytes of a split's partials), then wave 0 adds the waves' sums in wave
+// order: a fixed order, so results are identical from run to run.  (One wave per weight,
 // its lanes on 64 splits a whole partial array apart, read a cache line per
 // 4-byte value: 29.7 us for 85 splits of 73728 weights.)
-__global__ void __launch_bounds__(256) wgrad_reduce(float* __restrict__ dw, const float* __restrict__ ws, size_t n,
-                                                    int splits) {
-    __shared__ float part[4][64];
+template <int GROUPS>
+__global__ void __launch_bounds__(64 * GROUPS) wgrad_reduce(float* __restrict__ dw, const float* __restrict__ ws, size_t n,
+                                                            int splits) {
+    __shared__ float part[GROUPS][64];
     const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
     const size_t i = (size_t)blockIdx.x * 64 + lane;
     float s = 0.0f;
-    if (i < n)
-        for (int k = g; k < splits; k += 4) s += ws[(size_t)k * n + i];
+    if (i < n) {
+        // four at a time, so that their loads are in flight together
+        const float* __restrict__ w = ws + i;
+        int k = g;
+        for (; k + 3 * GROUPS < splits; k += 4 * GROUPS) {
+            const float a = w[(size_t)k * n], b = w[(size_t)(k + GROUPS) * n];
+            const float c = w[(size_t)(k + 2 * GROUPS) * n], d = w[(size_t)(k + 3 * GROUPS) * n];
+            s += (a + b) + (c + d);
+        }
+        for (; k < splits; k += GROUPS) s += w[(size_t)k * n];
+    }
     part[g][lane] = s;
     __syncthreads();
-    if (g == 0 && i < n) dw[i] = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+    if (g == 0 && i < n) {
+        float t = part[0][lane];
+#pragma unroll
+        for (int q = 1; q < GROUPS; ++q) t += part[q][lane];
+        dw[i] = t;
+    }
+}
+
+int launch_wgrad_reduce(lancius_hip_ctx* ctx, float* dw, const float* ws, size_t n, int splits) {
+    LANCIUS_REQUIRE((n + 63) / 64 < kMaxGridX, LANCIUS_HIP_ERR_SHAPE, "conv2d_bwd_weight: %zu weights", n);
+    // eight waves a workgroup from 16 splits on (32 x 3 -> 16 channels, 5x5, 256
+    // splits of 1200 weights: the reduction's loads were a chain of 64, 9.6 us);
+    // with fewer most of them would idle (N8 240->176 7x7, 3 splits of 2 M
+    // weights: 52 us with four, 63 with eight)
+    const dim3 grid((unsigned)((n + 63) / 64));
+    if (splits >= 16)
+        hipLaunchKernelGGL(wgrad_reduce<8>, grid, dim3(512), 0, ctx->stream, dw, ws, n, splits);
+    else
+        hipLaunchKernelGGL(wgrad_reduce<4>, grid, dim3(256), 0, ctx->stream, dw, ws, n, splits);
+    return check_launch("conv2d_wgrad_reduce");
 }
 
 template <int BM, int BN, int KH_T, int KW_T>
@@ -1223,6 +1252,20 @@ int launch_tile(lancius_hip_ctx* ctx, ConvParams& p, int tile) {
     }
 }
 
+// The fp32 weight gradient's time in us: 16-pixel k-tiles of 128 x 64 (64 x 64)
+// tiles, three workgroups a CU and at least 256 pixels each, then the sum of
+// the splits.  Fitted with wgrad_split_plan's to 90 shapes: N32 64->128 56^2
+// 144 (split products 103), N32 256->256 14^2 87 (58), N2 64->64 56^2 17 (17),
+// N5 112->160 1x1 at stride 2 of 11x8 10 (16).
+double wgrad_fp32_us(size_t C_out, size_t J, size_t P, bool direct) {
+    const double wide = C_out > 64 ? 1.0 : 0.62;
+    const double tiles = std::ceil(C_out / (C_out > 64 ? 128.0 : 64.0)) * std::ceil(J / 64.0);
+    const double splits = std::max(1.0, std::min(std::floor(768.0 / tiles), std::floor(P / 256.0)));
+    const double kt = std::ceil(P / splits / 16.0);
+    const double us = 4.5 + 0.58 * wide * kt * std::max(0.55, tiles * splits / 256) + (splits > 1 ? 6.5 : 0.0);
+    return direct ? us : 5.0 + 1.6 * us;  // images of a pixel count that is no multiple of 4: the staged kernel
+}
+
 }  // namespace
 }  // namespace lancius
 
@@ -1387,6 +1430,24 @@ extern "C" int lancius_hip_conv2d_bwd_weight_f32(lancius_hip_ctx* ctx, float* dw
     const size_t J = C_in * K_h * K_w;
     if (C_out * J == 0) return ok();
     if (int rc = bind_device(ctx)) return rc;
+    WgradSplitParams sp{dw, dy, x, (int)N, (int)C_in, (int)H, (int)W, (int)C_out, (int)H_out, (int)W_out, (int)K_h, (int)K_w,
+                        (int)stride, (int)pad, (int)J, 0, 0, 0, 0, 0, 0};
+    if (N > 0 && H_out > 0 && W_out > 0 && H > 0 && W > 0 && N * C_in < ((size_t)1 << 30) && N * C_out < ((size_t)1 << 30) &&
+        stride < (1u << 15) && pad < (1u << 15) && wgrad_split_fits(sp)) {
+        double us = 0.0;
+        wgrad_split_plan(sp, (size_t)cu_count(ctx), &us);
+        if (us < 1.15 * wgrad_fp32_us(C_out, J, N * H_out * W_out, H_out * W_out % 4 == 0 && H_out * W_out >= 16)) {
+            if (sp.splits > 1) {
+                void* ws = nullptr;
+                if (int rc = workspace(ctx, (size_t)sp.splits * C_out * J * sizeof(float), &ws)) return rc;
+                sp.out = (float*)ws;
+            }
+            if (int rc = launch_wgrad_split(ctx, sp)) return rc;
+            if (sp.splits > 1)
+                if (int rc = launch_wgrad_reduce(ctx, dw, sp.out, C_out * J, sp.splits)) return rc;
+            return ok();
+        }
+    }
     // 128 x 64 tiles (two 32 x 32 MFMA blocks per wave) when C_out > 64,
     // else 64 x 64 (one)
     const int BM = C_out > 64 ? 128 : 64, BN = 64;
@@ -1456,12 +1517,7 @@ extern "C" int lancius_hip_conv2d_bwd_weight_f32(lancius_hip_ctx* ctx, float* dw
     else
         hipLaunchKernelGGL((conv2d_wgrad_mfma<64, 64, bk>), grid, dim3(256), 0, ctx->stream, p);
     if (int rc = check_launch("conv2d_wgrad_mfma")) return rc;
-    if (p.splits > 1) {
-        const size_t n = C_out * J;
-        LANCIUS_REQUIRE((n + 63) / 64 < kMaxGridX, LANCIUS_HIP_ERR_SHAPE, "conv2d_bwd_weight: %zu weights", n);
-        hipLaunchKernelGGL(wgrad_reduce, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, ctx->stream, dw,
-                           (const float*)p.ws, n, p.splits);
-        if (int rc = check_launch("conv2d_wgrad_reduce")) return rc;
-    }
+    if (p.splits > 1)
+        if (int rc = launch_wgrad_reduce(ctx, dw, p.ws, C_out * J, p.splits)) return rc;
     return ok();
 }

@@ -27,4 +27,24 @@ size_t conv_split_tiles(const ConvSplitParams& p);  // workgroups of the launch
 // w: the filter [out][in][KH][KW] to lay out first (null: p.wt is ready).
 int launch_conv_split(lancius_hip_ctx* ctx, ConvSplitParams& p, const float* w);
 
+// The split-product weight gradient (wgrad_split.hip): ws gets `splits` partial
+// gradients [C_out][C_in KH KW], or dw the whole one when splits is 1.
+struct WgradSplitParams {
+    float* out;
+    const float* dy;
+    const float* x;
+    int N, C_in, H, W, C_out, Ho, Wo, KH, KW, stride, pad;
+    int J;          // C_in KH KW
+    int row_oct;    // octets of 8 output pixels in a row, the last one padded
+    int octets;     // N Ho row_oct
+    int chunk;      // k-steps (two octets) per split
+    int splits;
+    uint32_t tiles_m, tiles_n;
+};
+// Sizes within its 32-bit offsets.
+bool wgrad_split_fits(const WgradSplitParams& p);
+// Sets chunk and splits for a grid of about one workgroup per CU; us: an estimate of the launch.
+void wgrad_split_plan(WgradSplitParams& p, size_t cus, double* us);
+int launch_wgrad_split(lancius_hip_ctx* ctx, WgradSplitParams& p);
+
 }  // namespace lancius

@@ -1,0 +1,85 @@
+"""The split-product weight gradient (lancius_amd/csrc/wgrad_split.hip): row
+widths around the octets of 8 pixels, channel and tap counts at the edges of
+its tiles, strides, and non-finite inputs, against fp64."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import oracle
+from lancius_amd import prng
+from tests.conftest import case
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dev, x, dy, KH, KW, stride, pad):
+    N, C_in, H, W = x.shape
+    _, C_out, Ho, Wo = dy.shape
+    n = C_out * C_in * KH * KW
+    dx, dg, do = dev.upload(x), dev.upload(dy), dev.alloc(4 * n + 4096)
+    dev.fill(do, 7.0, n + 1024)
+    dev.conv2d_bwd_weight(do, dg, dx, N, C_in, H, W, C_out, Ho, Wo, KH, KW, stride, pad)
+    got = dev.download(do, (n + 1024,))
+    assert (got[n:] == 7.0).all()  # nothing is stored past the gradient
+    for b in (dx, dg, do):
+        b.free()
+    return got[:n].reshape(C_out, C_in, KH, KW)
+
+
+def _ref(x, dy, KH, KW, stride, pad):
+    w = torch.zeros(dy.shape[1], x.shape[1], KH, KW, dtype=torch.float64, requires_grad=True)
+    F.conv2d(torch.from_numpy(x).double(), w, None, stride, pad).backward(torch.from_numpy(dy).double())
+    return w.grad.numpy()
+
+
+def _inputs(seed, N, C_in, H, W, C_out, KH, KW, stride, pad):
+    Ho, Wo = (H + 2 * pad - KH) // stride + 1, (W + 2 * pad - KW) // stride + 1
+    return prng.normal(seed, (N, C_in, H, W)), prng.normal(seed + 1, (N, C_out, Ho, Wo), std=0.1)
+
+
+# (N, C_in, H, W, C_out, KH, KW, stride, pad)
+SHAPES = [
+    (16, 64, 40, 40, 128, 3, 3, 1, 1),      # whole octets
+    (9, 33, 41, 63, 72, 3, 3, 1, 1),        # rows of 63: the last octet one short
+    (8, 48, 37, 65, 160, 5, 5, 1, 2),       # rows of 65: an octet of one pixel
+    (6, 24, 50, 57, 130, 3, 5, 1, 2),       # an oblong filter, two channels over
+    (12, 40, 45, 33, 60, 5, 5, 2, 2),       # stride 2, 64-channel tiles
+    (4, 21, 35, 35, 70, 7, 7, 1, 3),
+    (8, 96, 29, 31, 96, 1, 1, 1, 0),
+    (3, 80, 64, 50, 144, 3, 3, 3, 0),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])
+def test_wgrad_split_shapes(dev, shape):
+    case(f"wgrad split {shape}")
+    x, dy = _inputs(7000, *shape)
+    geometry = shape[5:]
+    assert oracle.normwise_error(_run(dev, x, dy, *geometry), _ref(x, dy, *geometry)) <= oracle.tolerance(dy[0, 0].size * shape[0])
+
+
+def test_wgrad_split_is_repeatable(dev):
+    shape = (9, 33, 41, 63, 72, 3, 3, 1, 1)
+    x, dy = _inputs(7100, *shape)
+    assert np.array_equal(_run(dev, x, dy, 3, 3, 1, 1), _run(dev, x, dy, 3, 3, 1, 1))
+
+
+@pytest.mark.parametrize("stride", [1, 2])
+def test_wgrad_split_non_finite(dev, stride):
+    """An infinite or NaN pixel reaches the taps that see it, and no others."""
+    shape = (16, 64, 41, 40, 128, 3, 3, stride, 1)
+    case(f"wgrad split non-finite stride {stride}")
+    x, dy = _inputs(7200, *shape)
+    x[0, 3, 0, 0], x[5, 20, 17, 18] = np.inf, np.nan
+    dy[7, 9, 4, 5] = -np.inf
+    x[3, 50, 11, 12] = np.float32(3.4e38)  # rounds to infinity as bf16
+    got, ref = _run(dev, x, dy, 3, 3, stride, 1), _ref(x, dy, 3, 3, stride, 1)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(got[inf], ref[inf].astype(np.float32))
+    big = np.isfinite(ref) & (np.abs(ref) > 1e20)
+    assert big.any()
+    for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
+        err = oracle.normwise_error(np.where(part, got, 0).astype(np.float64) * scale, np.where(part, ref, 0) * scale)
+        assert err <= oracle.tolerance(dy[0, 0].size * 16)
