@@ -57,30 +57,58 @@ __global__ void __launch_bounds__(kThreads) sum_finish(float* __restrict__ out, 
     if (threadIdx.x == 0) out[0] = (float)s;
 }
 
-// SUM_AXIS0 over rows [r0, r1) of split blockIdx.y: one column per thread,
-// consecutive threads on consecutive columns (coalesced rows).
-__global__ void __launch_bounds__(kThreads) sum_axis0_split(float* __restrict__ out, double* __restrict__ partial,
-                                                            const float* __restrict__ in, size_t rows, size_t cols,
-                                                            size_t rchunk) {
-    const size_t c = (size_t)blockIdx.x * kThreads + threadIdx.x;
-    if (c >= cols) return;
+// SUM_AXIS0 over rows [r0, r1) of split blockIdx.y (T: the values, or the
+// splits' partial sums).  A workgroup takes w columns (16, 32 or 64: rows of
+// few columns still fill its waves); its 512 / w row groups each add every
+// (512 / w)-th row, eight loads in flight, and are then added in a fixed
+// order, in the wave by shuffles and over the eight waves through LDS.
+// Bound by the loads' latency: one column per thread over all rows of a split
+// was a chain of 64 to 512 dependent adds behind single loads (64 x 128:
+// 7.3 us a call, now 3.9; 512 x 128 49 us, now 5.8; 2048 x 4096 29, now 9.5).
+constexpr int kAxis0Threads = 512;
+constexpr int kAxis0Unroll = 8;
+template <typename T>
+__global__ void __launch_bounds__(kAxis0Threads) sum_axis0(float* __restrict__ out, double* __restrict__ partial,
+                                                           const T* __restrict__ in, size_t rows, size_t cols,
+                                                           size_t rchunk, int w) {
+    __shared__ double part[kAxis0Threads];
+    const size_t groups = kAxis0Threads / w;
     const size_t r0 = (size_t)blockIdx.y * rchunk;
     const size_t r1 = std::min(rows, r0 + rchunk);
-    double t = 0.0;
-    for (size_t r = r0; r < r1; ++r) t += (double)in[r * cols + c];
-    if (gridDim.y == 1)
-        out[c] = (float)t;
-    else
-        partial[(size_t)blockIdx.y * cols + c] = t;
+    for (size_t c0 = (size_t)blockIdx.x * w; c0 < cols; c0 += (size_t)gridDim.x * w) {
+        const size_t c = c0 + (threadIdx.x & (w - 1));
+        const T* __restrict__ x = in + std::min(c, cols - 1);
+        double t = 0.0;
+        for (size_t r = r0 + threadIdx.x / w; r < r1; r += kAxis0Unroll * groups) {
+            T v[kAxis0Unroll];
+#pragma unroll
+            for (int i = 0; i < kAxis0Unroll; ++i) v[i] = x[std::min(r + i * groups, r1 - 1) * cols];
+#pragma unroll
+            for (int i = 0; i < kAxis0Unroll; ++i) t += r + i * groups < r1 ? (double)v[i] : 0.0;
+        }
+        for (int off = w; off < 64; off <<= 1) t += __shfl_xor(t, off);
+        part[threadIdx.x] = t;
+        __syncthreads();
+        if ((int)threadIdx.x < w && c < cols) {
+            t = 0.0;
+#pragma unroll
+            for (int i = 0; i < kAxis0Threads; i += 64) t += part[threadIdx.x + i];
+            if (gridDim.y == 1)
+                out[c] = (float)t;
+            else
+                partial[(size_t)blockIdx.y * cols + c] = t;
+        }
+        __syncthreads();
+    }
 }
 
-__global__ void __launch_bounds__(kThreads) sum_axis0_finish(float* __restrict__ out,
-                                                             const double* __restrict__ partial, size_t cols,
-                                                             int splits) {
+// SUM_AXIS0 of a few rows: a column per thread.
+__global__ void __launch_bounds__(kThreads) sum_axis0_columns(float* __restrict__ out, const float* __restrict__ in,
+                                                              int rows, size_t cols) {
     const size_t c = (size_t)blockIdx.x * kThreads + threadIdx.x;
     if (c >= cols) return;
     double t = 0.0;
-    for (int s = 0; s < splits; ++s) t += partial[(size_t)s * cols + c];
+    for (int r = 0; r < rows; ++r) t += (double)in[(size_t)r * cols + c];
     out[c] = (float)t;
 }
 
@@ -146,25 +174,35 @@ int lancius_hip_sum_axis0_f32(lancius_hip_ctx* ctx, float* out, const float* in,
     LANCIUS_REQUIRE(ctx && out && in, LANCIUS_HIP_ERR_NULL_PTR, "sum_axis0: NULL argument");
     if (cols == 0) return ok();
     if (int rc = bind_device(ctx)) return rc;
-    const size_t col_blocks = (cols + kThreads - 1) / kThreads;
-    LANCIUS_REQUIRE(col_blocks < kMaxGridX, LANCIUS_HIP_ERR_SHAPE, "sum_axis0: %zu columns", cols);
-    // Row splits: ~1024 workgroups in all, each over >= 16 rows; none below
-    // 512 rows, where one pass is latency-bound anyway and a second launch
-    // would cost more than it saves.
-    size_t splits = rows <= 512 ? 1 : std::max<size_t>(1, std::min<size_t>((rows + 15) / 16, 1024 / col_blocks));
+    LANCIUS_REQUIRE((cols + kThreads - 1) / kThreads < kMaxGridX, LANCIUS_HIP_ERR_SHAPE, "sum_axis0: %zu columns", cols);
+    // Few rows with columns enough for one each per thread: no partial sums
+    // to add (16 x 2^20: 13.6 us, 40 with sum_axis0; 33 x 2^17: 5.0, 6.8; 64 x 2^18:
+    // 20.3, 11.5).
+    if (rows <= 48 && cols >= (1u << 16)) {
+        hipLaunchKernelGGL(sum_axis0_columns, dim3((unsigned)((cols + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                           ctx->stream, out, in, (int)rows, cols);
+        return check_launch("sum_axis0_columns");
+    }
+    const int w = cols <= 16 ? 16 : cols <= 32 ? 32 : 64;
+    const size_t col_blocks = (cols + w - 1) / w, groups = kAxis0Threads / w;
+    // Row splits: ~1024 workgroups in all, each thread over >= 16 rows; none
+    // while a thread has up to 64, where a second launch would cost more than
+    // it saves (512 x 128: 5.8 us in one, 513 x 128 6.5 in two).
+    size_t splits = rows <= 64 * groups ? 1 : std::max<size_t>(1, std::min<size_t>(rows / (16 * groups), 1024 / col_blocks));
     splits = std::min<size_t>(splits, 65535);
     const size_t rchunk = rows ? (rows + splits - 1) / splits : 1;
     splits = rows ? (rows + rchunk - 1) / rchunk : 1;
+    const unsigned grid_x = (unsigned)std::min<size_t>(col_blocks, 1u << 22);  // 2^31 work-items
     double* ws = nullptr;
     if (splits > 1)
         if (int rc = workspace(ctx, splits * cols * sizeof(double), (void**)&ws)) return rc;
-    hipLaunchKernelGGL(sum_axis0_split, dim3((unsigned)col_blocks, (unsigned)splits), dim3(kThreads), 0, ctx->stream,
-                       out, ws, in, rows, cols, rchunk);
-    if (int rc = check_launch("sum_axis0_split")) return rc;
+    hipLaunchKernelGGL(sum_axis0<float>, dim3(grid_x, (unsigned)splits), dim3(kAxis0Threads), 0,
+                       ctx->stream, out, ws, in, rows, cols, rchunk, w);
+    if (int rc = check_launch("sum_axis0")) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(sum_axis0_finish, dim3((unsigned)col_blocks), dim3(kThreads), 0, ctx->stream, out,
-                           (const double*)ws, cols, (int)splits);
-        if (int rc = check_launch("sum_axis0_finish")) return rc;
+        hipLaunchKernelGGL(sum_axis0<double>, dim3(grid_x), dim3(kAxis0Threads), 0, ctx->stream, out,
+                           nullptr, (const double*)ws, splits, cols, splits, w);
+        if (int rc = check_launch("sum_axis0")) return rc;
     }
     return ok();
 }

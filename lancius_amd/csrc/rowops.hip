@@ -305,6 +305,127 @@ __global__ void __launch_bounds__(kRowThreads) softmax_bwd_rows(float* __restric
     for (int c = lane; c < cols; c += 64) out[base + c] = y[base + c] * (dy[base + c] - dot);
 }
 
+// The loss gives a row to L lanes (64 / L rows a wave: classes
+// are few), which keep its logits and targets in NV registers each; NV = 0: a
+// wave per row that reads it again for each pass (more than 256 classes).
+// Bound by round trips to memory, not by bytes: 64 x 10 18.9 us in 16 rounds of
+// four waves, now 4.2 in one round; 512 x 100 181 us, now 6.7 in two launches.
+template <int L, int NV>
+struct CrossEntropyRow {
+    float m, s;  // row max, sum of exp(x - max)
+    float x[NV ? NV : 1], y[NV ? NV : 1];
+    const float *xr, *yr;
+    int cols, lane;
+    // row < rows; each lane of the wave calls it (rows past the end: clamped by the caller)
+    __device__ __forceinline__ CrossEntropyRow(const float* __restrict__ X, const float* __restrict__ Y, int row, int cols_)
+        : xr(X + (size_t)row * cols_), yr(Y + (size_t)row * cols_), cols(cols_), lane(threadIdx.x & (L - 1)) {
+        m = -INFINITY;
+        s = 0.0f;
+        if constexpr (NV != 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int c = min(lane + L * i, cols - 1);
+                x[i] = xr[c];
+                y[i] = yr[c];
+            }
+#pragma unroll
+            for (int i = 0; i < NV; ++i) m = lane + L * i < cols ? fmaxf(m, x[i]) : m;
+        } else {
+            for (int c = lane; c < cols; c += L) m = fmaxf(m, xr[c]);
+        }
+#pragma unroll
+        for (int off = L / 2; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+        if constexpr (NV != 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) s += lane + L * i < cols ? expf(x[i] - m) : 0.0f;
+        } else {
+            for (int c = lane; c < cols; c += L) s += expf(xr[c] - m);
+        }
+#pragma unroll
+        for (int off = L / 2; off >= 1; off >>= 1) s += __shfl_xor(s, off);
+    }
+    // sum over the entries with y == 1 of (x - logsumexp(x)), in fp64
+    // (lancius_scheduler.c:68-83)
+    __device__ __forceinline__ double term() const {
+        const double lse = (double)logf(s) + (double)m;
+        double t = 0.0;
+        each([&](int, float xv, float yv) {
+            if (yv == 1.0f) t += (double)xv - lse;
+        });
+#pragma unroll
+        for (int off = L / 2; off >= 1; off >>= 1) t += __shfl_xor(t, off);
+        return t;
+    }
+    template <typename F>
+    __device__ __forceinline__ void each(F&& f) const {
+        if constexpr (NV != 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                if (lane + L * i < cols) f(lane + L * i, x[i], y[i]);
+        } else {
+            for (int c = lane; c < cols; c += L) f(c, xr[c], yr[c]);
+        }
+    }
+};
+
+// CROSS_ENTROPY, first pass: each row's term.
+template <int L, int NV>
+__global__ void __launch_bounds__(kRowThreads) cross_entropy_rows(double* __restrict__ row_terms,
+                                                                  const float* __restrict__ x,
+                                                                  const float* __restrict__ y, int rows, int cols) {
+    const int row = blockIdx.x * (kRowThreads / L) + threadIdx.x / L;
+    const CrossEntropyRow<L, NV> r(x, y, min(row, rows - 1), cols);
+    const double t = r.term();
+    if (row < rows && r.lane == 0) row_terms[row] = t;
+}
+
+// Sum of the workgroup's values in a fixed order, valid in thread 0.
+template <int THREADS>
+__device__ __forceinline__ double block_sum(double t) {
+    __shared__ double part[THREADS / 64];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) t += __shfl_xor(t, off);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = t;
+    __syncthreads();
+    t = 0.0;
+#pragma unroll
+    for (int w = 0; w < THREADS / 64; ++w) t += part[w];
+    return t;
+}
+
+// One workgroup does both passes, so the loss is one launch; its rows are
+// taken kLossThreads / L at a time.
+constexpr int kLossThreads = 1024;
+template <int L, int NV>
+__global__ void __launch_bounds__(kLossThreads) cross_entropy_small(float* __restrict__ out, const float* __restrict__ x,
+                                                                    const float* __restrict__ y, int rows, int cols) {
+    double acc = 0.0;
+    for (int base = 0; base < rows; base += kLossThreads / L) {
+        const int row = base + threadIdx.x / L;
+        const CrossEntropyRow<L, NV> r(x, y, min(row, rows - 1), cols);
+        const double t = r.term();
+        acc += row < rows && r.lane == 0 ? t : 0.0;
+    }
+    const double total = block_sum<kLossThreads>(acc);
+    if (threadIdx.x == 0) out[0] = (float)fabs(-total / (double)rows);
+}
+
+// Second pass: out[0] = |-(sum of row terms) / rows| (:84-85), summed by one
+// workgroup in a fixed order, eight loads in flight a thread.
+__global__ void __launch_bounds__(kLossThreads) cross_entropy_finish(float* __restrict__ out,
+                                                                     const double* __restrict__ row_terms, int rows) {
+    double t = 0.0;
+    for (int r = threadIdx.x; r < rows; r += 8 * kLossThreads) {
+        double v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = row_terms[min(r + i * kLossThreads, rows - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t += r + i * kLossThreads < rows ? v[i] : 0.0;
+    }
+    const double total = block_sum<kLossThreads>(t);
+    if (threadIdx.x == 0) out[0] = (float)fabs(-total / (double)rows);
+}
+
 // Row max and sum of exp(x - max) of one row, for one wave.
 __device__ __forceinline__ void row_lse_parts(const float* __restrict__ x, int cols, int lane, float& m, float& s) {
     m = -INFINITY;
@@ -313,72 +434,6 @@ __device__ __forceinline__ void row_lse_parts(const float* __restrict__ x, int c
     s = 0.0f;
     for (int c = lane; c < cols; c += 64) s += expf(x[c] - m);
     s = wave_sum(s);
-}
-
-// CROSS_ENTROPY, first pass (lancius_scheduler.c:68-83): per row,
-// sum over the entries with y == 1 of (x - logsumexp(x)), in fp64.
-__global__ void __launch_bounds__(kRowThreads) cross_entropy_rows(double* __restrict__ row_terms,
-                                                                  const float* __restrict__ x,
-                                                                  const float* __restrict__ y, int rows, int cols) {
-    const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (row >= rows) return;
-    const float* xr = x + (size_t)row * cols;
-    const float* yr = y + (size_t)row * cols;
-    float m, s;
-    row_lse_parts(xr, cols, lane, m, s);
-    const double lse = (double)logf(s) + (double)m;
-    double t = 0.0;
-    for (int c = lane; c < cols; c += 64)
-        if (yr[c] == 1.0f) t += (double)xr[c] - lse;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) t += __shfl_xor(t, off);
-    if (lane == 0) row_terms[row] = t;
-}
-
-// Up to 4096 rows: one workgroup does both passes (each wave takes rows
-// w, w+4, ...), so the loss is one launch.
-__global__ void __launch_bounds__(kRowThreads) cross_entropy_small(float* __restrict__ out, const float* __restrict__ x,
-                                                                   const float* __restrict__ y, int rows, int cols) {
-    __shared__ double part[kRowsPerBlock];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double acc = 0.0;  // this wave's rows, in row order
-    for (int row = wave; row < rows; row += kRowsPerBlock) {
-        const float* xr = x + (size_t)row * cols;
-        const float* yr = y + (size_t)row * cols;
-        float m, s;
-        row_lse_parts(xr, cols, lane, m, s);
-        const double lse = (double)logf(s) + (double)m;
-        double t = 0.0;
-        for (int c = lane; c < cols; c += 64)
-            if (yr[c] == 1.0f) t += (double)xr[c] - lse;
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) t += __shfl_xor(t, off);
-        acc += t;
-    }
-    if (lane == 0) part[wave] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double total = 0.0;
-        for (int w = 0; w < kRowsPerBlock; ++w) total += part[w];
-        out[0] = (float)fabs(-total / (double)rows);
-    }
-}
-
-// Second pass: out[0] = |-(sum of row terms) / rows| (:84-85), summed by one
-// workgroup in a fixed order.
-__global__ void __launch_bounds__(256) cross_entropy_finish(float* __restrict__ out,
-                                                            const double* __restrict__ row_terms, int rows) {
-    __shared__ double part[256];
-    double t = 0.0;
-    for (int r = threadIdx.x; r < rows; r += 256) t += row_terms[r];
-    part[threadIdx.x] = t;
-    __syncthreads();
-    for (int w = 128; w >= 1; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = (float)fabs(-part[0] / (double)rows);
 }
 
 // CROSS_ENTROPY_BWD (lancius_scheduler.c:89-104):
@@ -396,6 +451,21 @@ __global__ void __launch_bounds__(kRowThreads) cross_entropy_bwd_rows(float* __r
     row_lse_parts(x + base, cols, lane, m, s);
     const float scale = (float)((double)g[0] / (double)rows);
     for (int c = lane; c < cols; c += 64) out[base + c] = (expf(x[base + c] - m) / s - y[base + c]) * scale;
+}
+
+// f(lanes a row, values a lane): the narrowest of the kernels' forms that
+// holds a row of cols.
+template <typename F>
+void with_row_form(size_t cols, F&& f) {
+    using std::integral_constant;
+    if (cols <= 16)
+        f(integral_constant<int, 16>{}, integral_constant<int, 1>{});
+    else if (cols <= 64)
+        f(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+    else if (cols <= 256)
+        f(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+    else
+        f(integral_constant<int, 64>{}, integral_constant<int, 0>{});
 }
 
 // RMSNorm (lancius_kernels.c:381-396): out = x * (1 / sqrt(mean(x^2) + eps)) * gamma.
@@ -796,17 +866,29 @@ int lancius_hip_cross_entropy_f32(lancius_hip_ctx* ctx, float* out, const float*
     LANCIUS_REQUIRE(rows > 0 && cols > 0 && cols < (1u << 30) && rows < (1u << 30), LANCIUS_HIP_ERR_SHAPE,
                     "cross_entropy: rows=%zu cols=%zu", rows, cols);
     if (int rc = bind_device(ctx)) return rc;
-    if (rows <= 4096) {
-        hipLaunchKernelGGL(cross_entropy_small, dim3(1), dim3(kRowThreads), 0, ctx->stream, out, x, y, (int)rows,
-                           (int)cols);
-        return check_launch("cross_entropy_small");
-    }
+    // One launch while its workgroup has few rounds of rows (64 at a time of
+    // up to 16 classes, 16 of more); two launches take 6.7 us.  256 x 10 in 4
+    // rounds: 5.1; 64 x 100 in 4: 7.8; 32 x 1000 in 2: 16.
+    const size_t round = kLossThreads / (cols <= 16 ? 16 : 64);
+    // Up to 4096 rows need no scratch memory: a capture that has none yet
+    // (it cannot allocate) records the one launch.
+    const bool one = rows <= round * (cols <= 16 ? 4 : cols <= 256 ? 2 : 1) ||
+                     (rows <= 4096 && ctx->capturing && ctx->workspace_bytes < rows * sizeof(double));
     void* ws = nullptr;
-    if (int rc = workspace(ctx, rows * sizeof(double), &ws)) return rc;
-    hipLaunchKernelGGL(cross_entropy_rows, dim3(ceil_div(rows, kRowsPerBlock)), dim3(kRowThreads), 0, ctx->stream,
-                       (double*)ws, x, y, (int)rows, (int)cols);
-    if (int rc = check_launch("cross_entropy_rows")) return rc;
-    hipLaunchKernelGGL(cross_entropy_finish, dim3(1), dim3(256), 0, ctx->stream, out, (const double*)ws, (int)rows);
+    if (!one)
+        if (int rc = workspace(ctx, rows * sizeof(double), &ws)) return rc;
+    with_row_form(cols, [&](auto l, auto nv) {
+        constexpr int L = decltype(l)::value, NV = decltype(nv)::value;
+        if (one)
+            hipLaunchKernelGGL((cross_entropy_small<L, NV>), dim3(1), dim3(kLossThreads), 0, ctx->stream, out, x, y,
+                               (int)rows, (int)cols);
+        else
+            hipLaunchKernelGGL((cross_entropy_rows<L, NV>), dim3(ceil_div(rows, kRowThreads / L)), dim3(kRowThreads), 0,
+                               ctx->stream, (double*)ws, x, y, (int)rows, (int)cols);
+    });
+    if (int rc = check_launch("cross_entropy")) return rc;
+    if (one) return ok();
+    hipLaunchKernelGGL(cross_entropy_finish, dim3(1), dim3(kLossThreads), 0, ctx->stream, out, (const double*)ws, (int)rows);
     return check_launch("cross_entropy_finish");
 }
 
