@@ -33,7 +33,7 @@ ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 HIPCC = str(ROCM / "bin" / "hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["capi.hip", "gemm.hip", "gemm_split.hip", "attention.hip", "attention_split.hip",
+HIP_SOURCES = ["capi.hip", "gemm.hip", "gemm_small.hip", "gemm_split.hip", "attention.hip", "attention_split.hip",
                "conv.hip", "conv_split.hip", "wgrad_split.hip", "rowops.hip", "reduce.hip", "pool.hip",
                "int8.hip", "io.hip", "chain.hip", "probe.hip", "basis.hip"]
 HOST_C_SOURCES = ["host/graph_ir.c", "host/graph_plan.c", "host/graph_autodiff.c", "host/graph_io.c",

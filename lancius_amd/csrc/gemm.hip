@@ -1242,6 +1242,15 @@ GemmPlan gemm_plan(size_t count, size_t M, size_t K, size_t N, bool plain, bool 
     return best;
 }
 
+// The skinny kernel's time in us: a launch, then what one workgroup takes for
+// its K slice and the adding of slices; scalar rows of B (N % 4) slow it down.
+double skinny_us(size_t count, size_t M, size_t K, size_t N, bool vb) {
+    const double k = (double)K, bytes = 4.0 * (double)count * k * N;
+    const double us = vb ? (M <= 16 ? (K <= 512 ? 4.9 : K <= 1664 && N <= 64 ? 5.8 : 6.3) : (K <= 512 ? 7.0 : 8.7))
+                         : (M <= 16 ? 6.0 + std::min(5.0, 0.010 * k) : 8.0 + std::min(7.0, 0.014 * k));
+    return std::max(us, 3.0 + bytes / 4e6);
+}
+
 // fixed: when not null, split-K partials and arrival counters go to its
 // buffers instead of the context's, and nothing is allocated.
 int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const float* const* A,
@@ -1298,13 +1307,25 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
     p.K = (int)K;
     p.act = act;
 
+    const size_t big_tiles = count * ((M + 127) / 128) * ((N + 127) / 128);
+    // 32-bit buffer offsets (gemm_split.hip, gemm_small.hip)
+    const bool split_fits = (M + 96) * (K + 96) * sizeof(float) < kSplitMaxBytes &&
+                            (K + 96) * (N + 96) * sizeof(float) < kSplitMaxBytes &&
+                            (M + 256) * (N + 256) * sizeof(float) < kSplitMaxBytes;
+    const SmallPlan small_plan = split_fits ? gemm_small_plan(count, M, K, N, tb) : SmallPlan{16, 1e30};
+    auto run_small = [&] {
+        if (int rc = launch_gemm_small(ctx, p, (int)count, ta, tb, small_plan.tile)) return rc;
+        return ok();
+    };
     // M <= 32 (B not transposed): the B-streaming skinny kernel, one
     // workgroup per (64 columns, 64 x waves K rows), the K slices added
     // inside the launch.  Measured on MI355X it beats the tiled kernel up to
     // M = 32 (16x4096x4096: 22 vs 34 us with the first skinny design;
     // 32x2048x120: 10.6 vs 13.6 us) and loses at M = 64 with four row tiles
-    // (64x4096x4096: 43 vs 38 us; 64x784x256: 13.0 vs 11.8 us).
+    // (64x4096x4096: 43 vs 38 us; 64x784x256: 13.0 vs 11.8 us).  Where little
+    // of B is read, small tiles are ahead (5x536x3665: 12.4 -> 4.9 us).
     if (M <= 32 && !tb) {
+        if (small_plan.us < skinny_us(count, M, K, N, vb)) return run_small();
         const int mt = M <= 16 ? 1 : 2;
         const size_t splits = (K + 64 * kSkinnyWaves - 1) / (64 * kSkinnyWaves);
         const size_t col_blocks = (N + 63) / 64;
@@ -1330,15 +1351,12 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
         }
     }
 
-    const size_t big_tiles = count * ((M + 127) / 128) * ((N + 127) / 128);
+    const GemmPlan plan = gemm_plan(count, M, K, N, !ta && !tb, vec);
+    if (small_plan.us < plan.us) return run_small();
     // Products large enough for the bf16 matrix cores' split products
     // (gemm_split.hip); both operands transposed, or one beyond 32-bit
     // offsets, stay with the fp32 kernels.
-    const bool split_fits = (M + 96) * (K + 96) * sizeof(float) < kSplitMaxBytes &&
-                            (K + 96) * (N + 96) * sizeof(float) < kSplitMaxBytes &&
-                            (M + 256) * (N + 256) * sizeof(float) < kSplitMaxBytes;
     if (!(ta && tb) && split_fits && (K >= 32 || big_tiles >= 768)) {
-        const GemmPlan plan = gemm_plan(count, M, K, N, !ta && !tb, vec);
         if (plan.tile >= 0) {
             const size_t steps = (K + 31) / 32, chunk = (steps + plan.splits - 1) / plan.splits;
             p.splits = (int)((steps + chunk - 1) / chunk);  // no empty K range

@@ -31,4 +31,13 @@ int launch_gemm_split(lancius_hip_ctx* ctx, GemmParams& p, int count, bool ta, b
 // 256 rows past C's.
 constexpr size_t kSplitMaxBytes = (size_t)1 << 31;
 
+// gemm_small.hip: the tile (16 or 32) and cost of a product in one launch of
+// small tiles, and that launch; operands and C within split_fits' bounds.
+struct SmallPlan {
+    int tile;
+    double us;
+};
+SmallPlan gemm_small_plan(size_t count, size_t M, size_t K, size_t N, bool tb);
+int launch_gemm_small(lancius_hip_ctx* ctx, GemmParams& p, int count, bool ta, bool tb, int tile);
+
 }  // namespace lancius
