@@ -51,6 +51,12 @@ int bind_device(lancius_hip_ctx* ctx);
 // its stream, so one buffer serves every kernel of the context.
 int workspace(lancius_hip_ctx* ctx, size_t bytes, void** out);
 
+// Whether workspace(ctx, bytes) would succeed now: during a capture nothing can
+// be allocated, and a kernel that needs less scratch memory is taken instead.
+inline bool workspace_ready(const lancius_hip_ctx* ctx, size_t bytes) {
+    return !ctx->capturing || bytes == 0 || (ctx->workspace && bytes <= ctx->workspace_bytes);
+}
+
 // Compute units of the context's device (cached in the context).
 int cu_count(lancius_hip_ctx* ctx);
 

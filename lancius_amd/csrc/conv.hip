@@ -1179,7 +1179,8 @@ int launch_tile(lancius_hip_ctx* ctx, ConvParams& p, int tile);
 // 512 (N32 64->128 56^2 99); 64 x 128 tiles 8 + 0.0235 K, 0.06 K a round of 512
 // (N32 128->64 56^2 123).
 double conv_split_us(const ConvSplitParams& sp) {
-    const double k = (double)sp.KH * sp.KW * sp.C16, t = (double)conv_split_tiles(sp);
+    const int s = sp.dgrad ? sp.stride : 1;
+    const double k = (double)((sp.KH + s - 1) / s) * ((sp.KW + s - 1) / s) * sp.C16, t = (double)conv_split_tiles(sp);
     const bool wide = sp.C_out > 64;
     if (t <= 256) return 8.0 + (wide ? 0.034 : 0.0235) * k;
     return 9.0 * std::max(1.0, t / 512) + (wide ? 0.0675 : 0.06) * k * std::max(0.8, t / 512);
@@ -1204,19 +1205,26 @@ double conv_fp32_us(const ConvParams& q) {
     return 4.5 + (wide ? 0.72 : 0.42) * kt / ways + 2.5 * (ways - 1);
 }
 
-// The convolution q as split products (conv_split.hip), where they are the
-// faster kernel (by the estimates, with a tenth to spare).
-bool use_split(const ConvParams& q, ConvSplitParams* sp) {
+// The convolution q as conv_split.hip's kernels, where they are the faster ones
+// (by the estimates; split products with a tenth to spare).
+bool use_split(lancius_hip_ctx* ctx, const ConvParams& q, ConvSplitParams* sp) {
     *sp = ConvSplitParams{q.out, q.in, q.wt, q.bias, q.N, q.C_in, (q.C_in + 15) / 16 * 16, q.H, q.W, q.C_out, q.KH, q.KW,
-                          q.stride, q.pad, q.Ho, q.Wo, 0, q.act, 0};
+                          q.stride, q.pad, q.Ho, q.Wo, 0, q.act, 0, 0};
     if (q.prep == 2) {  // the gradient of a convolution of stride 1
         sp->dgrad = 1;
         sp->pad = q.KH - 1 - q.pad;
     }
     if (!conv_split_fits(*sp)) return false;
+    if (q.prep != 0 && !workspace_ready(ctx, conv_split_weight_bytes(*sp))) return false;
     // (a ragged channel count has the filter laid out for the call, 4 us)
     const double prep = q.prep == 1 && (q.C_in % 16 != 0 || q.C_out % 4 != 0) ? 4.0 : 0.0;
-    return (conv_split_us(*sp) + prep) * 1.1 < conv_fp32_us(q);
+    const double split = (conv_split_us(*sp) + prep) * 1.1, fp32 = conv_fp32_us(q);
+    int tile;
+    if (conv_small_plan(*sp, &tile) + prep < std::min(split, fp32)) {
+        sp->small_tile = tile;
+        return true;
+    }
+    return split < fp32;
 }
 
 // One launch per run of images whose input stays under 2 GiB (the direct
@@ -1233,7 +1241,7 @@ int launch_batches(lancius_hip_ctx* ctx, const ConvParams& p, int tile) {
         q.out = p.out + n0 * img_out;
         q.Ptotal = (long long)q.N * p.Ho * p.Wo;
         ConvSplitParams sp{};
-        if (use_split(q, &sp)) {
+        if (use_split(ctx, q, &sp)) {
             if (int rc = launch_conv_split(ctx, sp, p.prep == 0 ? nullptr : p.prep == 2 ? p.w_src : p.w)) return rc;
             continue;
         }
@@ -1378,12 +1386,15 @@ extern "C" int lancius_hip_conv2d_bwd_input_f32(lancius_hip_ctx* ctx, float* dx,
                          H + 2 * pad + 1 == H_out + K_h && W + 2 * pad + 1 == W_out + K_w;
     if (!as_conv) {
         ConvSplitParams sp{dx, dy, nullptr, nullptr, (int)N, (int)C_out, (int)((C_out + 15) / 16 * 16), (int)H_out, (int)W_out,
-                           (int)C_in, (int)K_h, (int)K_w, (int)stride, (int)pad, (int)H, (int)W, 1, LANCIUS_HIP_ACT_NONE, 0};
+                           (int)C_in, (int)K_h, (int)K_w, (int)stride, (int)pad, (int)H, (int)W, 1, LANCIUS_HIP_ACT_NONE, 0, 0};
         // (up to a dozen products an element, or sizes beyond its offsets, the
         // split-product kernel leaves to the direct one: N15 4->8 1x1 107x11
         // 6.1 us against 8.6; N16 64->128 3x3 56^2 the other way, 3263
         // against 32)
-        if (C_out * K_h * K_w > 12 && stride <= 16 && K_h < (1u << 15) && K_w < (1u << 15) && C_out > 0 && pad < (1u << 30) && conv_split_fits(sp)) {
+        if (C_out * K_h * K_w > 12 && stride <= 16 && K_h < (1u << 15) && K_w < (1u << 15) && C_out > 0 && pad < (1u << 30) && conv_split_fits(sp) &&
+            workspace_ready(ctx, conv_split_weight_bytes(sp))) {
+            int tile;
+            if (conv_small_plan(sp, &tile) < conv_split_us(sp)) sp.small_tile = tile;
             const int rc = launch_conv_split(ctx, sp, w);
             return rc ? rc : ok();
         }
@@ -1436,7 +1447,8 @@ extern "C" int lancius_hip_conv2d_bwd_weight_f32(lancius_hip_ctx* ctx, float* dw
         stride < (1u << 15) && pad < (1u << 15) && wgrad_split_fits(sp)) {
         double us = 0.0;
         wgrad_split_plan(sp, (size_t)cu_count(ctx), &us);
-        if (us < 1.15 * wgrad_fp32_us(C_out, J, N * H_out * W_out, H_out * W_out % 4 == 0 && H_out * W_out >= 16)) {
+        if (workspace_ready(ctx, sp.splits > 1 ? (size_t)sp.splits * C_out * J * sizeof(float) : 0) &&
+            us < 1.15 * wgrad_fp32_us(C_out, J, N * H_out * W_out, H_out * W_out % 4 == 0 && H_out * W_out >= 16)) {
             if (sp.splits > 1) {
                 void* ws = nullptr;
                 if (int rc = workspace(ctx, (size_t)sp.splits * C_out * J * sizeof(float), &ws)) return rc;

@@ -20,7 +20,10 @@ struct ConvSplitParams {
     int N, C_in, C16, H, W, C_out, KH, KW, stride, pad, Ho, Wo;  // C16: C_in rounded up to 16
     int dgrad, act;
     uint32_t tiles_m;  // set by the launch
+    int small_tile;    // 16 or 32: conv2d_small's tile, 0: split products
 };
+// Time in us of the small-tile kernel with the better of its tiles.
+double conv_small_plan(const ConvSplitParams& p, int* tile);
 bool conv_split_fits(const ConvSplitParams& p);
 size_t conv_split_weight_bytes(const ConvSplitParams& p);
 size_t conv_split_tiles(const ConvSplitParams& p);  // workgroups of the launch

@@ -22,6 +22,7 @@
 // -> 114 us: 512 shares of 64 KB of sums).  64 x 128 tiles read 9 KB of operands
 // from LDS for 12 products a wave, 128 x 128 tiles 12 KB for 24.
 #include <algorithm>
+#include <cmath>
 
 #include "conv.hpp"
 #include "split_tile.hpp"
@@ -213,6 +214,121 @@ __global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, 2) conv2d_spl
     }
 }
 
+// The same product in fp32 for grids that leave most CUs idle: a tile of T
+// channels x T pixels per workgroup, K spread over its waves, operands loaded
+// straight into the matrix cores' registers (gemm_small.hip's scheme). What
+// bounds it is a wave's chain of gathers, what bounded the staged tiles the
+// same chain for 128 pixels with a barrier a step. Before and now: N32 16->32
+// 5x5 16^2 15.8, 5.5 us, its input gradient 28, 10.4; N1 64->128 3x3 56^2 23.5,
+// 9.6; N3 176->16 5x5 of 8x9 115, 14.
+template <int T, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) conv2d_small(const ConvSplitParams p) {
+    constexpr int NQ = T * T / 64;                // sums a lane holds
+    constexpr int KS = 4 * (64 / T);              // k of a group: four MFMAs
+    constexpr int NACC = T == 32 ? 2 : 4;
+    constexpr int kOut = 0x7ffffff0;
+    __shared__ float red[WAVES][NQ][64];
+    const ConvClass cl = conv_class(p, blockIdx.z);
+    const int pix_img = cl.th_n * cl.tw_n, P_n = p.N * pix_img;
+    const uint32_t tiles_n = (uint32_t)((P_n + T - 1) / T);
+    if (blockIdx.x >= p.tiles_m * tiles_n) return;  // a class of fewer pixels than the largest
+    const int m0 = (int)(blockIdx.x % p.tiles_m) * T, P0 = (int)(blockIdx.x / p.tiles_m) * T;
+    const int K = cl.kh * cl.kw * p.C16;
+    const int hw4 = p.H * p.W * 4;
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.wt + cl.w_off), 0, p.C_out * K * 4, kBufferRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.in), 0, p.N * p.C_in * hw4, kBufferRsrcWord3);
+    const int lane = threadIdx.x & 63, lr = lane % T, lk = lane / T;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+
+    // this lane's pixel
+    const int P = P0 + lr;
+    const bool valid = P < P_n;
+    const int n = P / pix_img, rem = P - n * pix_img, th = rem / cl.tw_n, tw = rem - th * cl.tw_n;
+    const int hb = cl.mul * th + cl.h0, wb = cl.mul * tw + cl.w0;
+    const int img = n * p.C_in * hw4;
+
+    // this wave's groups [gi, ge), the next one to load at (tap uh uw, channels c0..)
+    const int groups = K / KS, per = (groups + WAVES - 1) / WAVES;
+    int gi = wave * per;
+    const int ge = min(groups, gi + per);
+    int tap = gi * KS / p.C16, c0 = gi * KS - tap * p.C16, k0 = gi * KS;
+    int uh = cl.kw ? tap / cl.kw : 0, uw = tap - uh * cl.kw;
+    typedef float acc_t __attribute__((ext_vector_type(NQ)));
+    f32x4 a[2], b[2];
+    acc_t acc[NACC] = {};  // by k modulo NACC: short chains, and no MFMA waits for the one before
+    auto load = [&](int s) {
+        const int hi = hb + cl.dir * uh, wi = wb + cl.dir * uw, c = c0 + 4 * lk;
+        const bool in = valid & ((unsigned)hi < (unsigned)p.H) & ((unsigned)wi < (unsigned)p.W);
+        const int off = img + (hi * p.W + wi) * 4 + 4 * lk * hw4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)  // (channels past C_in are the next image's)
+            b[s][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                    rx, pick(in & (c + j < p.C_in), off, kOut), (c0 + j) * hw4, 0));
+        a[s] = __builtin_bit_cast(f32x4,
+                                  __builtin_amdgcn_raw_buffer_load_b128(rw, ((m0 + lr) * K + 4 * lk) * 4, k0 * 4, 0));
+        k0 += KS;
+        c0 += KS;
+        if (c0 == p.C16) {
+            c0 = 0;
+            if (++uw == cl.kw) {
+                uw = 0;
+                ++uh;
+            }
+        }
+    };
+    auto multiply = [&](int s) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            acc_t& c = acc[j % NACC];
+            if constexpr (T == 32)
+                c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[s][j], c, 0, 0, 0);
+            else
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][j], b[s][j], c, 0, 0, 0);
+        }
+    };
+    if (gi < ge) {
+        load(0);
+        for (; gi + 2 < ge; gi += 2) {
+            load(1);
+            multiply(0);
+            load(0);
+            multiply(1);
+        }
+        if (gi + 1 < ge) {
+            load(1);
+            multiply(0);
+            multiply(1);
+        } else {
+            multiply(0);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        float s = acc[0][q] + acc[1][q];
+        if constexpr (NACC == 4) s += acc[2][q] + acc[3][q];
+        red[wave][q][lane] = s;
+    }
+    __syncthreads();
+
+    // element (q, lane): pixel lane % T, channel 8 (q / 4) + 4 (lane / T) + q % 4
+    const int ohw = p.Ho * p.Wo;
+    float* __restrict__ out = p.out + (size_t)n * p.C_out * ohw + (cl.os * th + cl.oh0) * p.Wo + cl.os * tw + cl.ow0;
+    const bool relu = p.act == kActRelu;
+#pragma unroll
+    for (int q0 = 0; q0 < NQ; q0 += WAVES) {
+        const int q = q0 + wave, c = m0 + 8 * (q >> 2) + 4 * lk + (q & 3);
+        if (q < NQ && valid && c < p.C_out) {
+            float s = 0.0f;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) s += red[w][q][lane];
+            if (p.bias) s += p.bias[c];
+            out[(size_t)c * ohw] = relu ? relu_ref(s) : s;
+        }
+    }
+}
+
 // wt[channel][tap][C16]: the forward filter re-laid, channels past C_in zero.
 __global__ void __launch_bounds__(256) conv_split_weights(float* __restrict__ wt, const float* __restrict__ w, int C_out,
                                                           int C_in, int C16, int KHW) {
@@ -257,6 +373,14 @@ int launch(lancius_hip_ctx* ctx, ConvSplitParams& p, size_t P_max, unsigned clas
     return check_launch("conv2d_split");
 }
 
+template <int T, int WAVES>
+int launch_small(lancius_hip_ctx* ctx, ConvSplitParams& p, size_t P_max, unsigned classes) {
+    p.tiles_m = (uint32_t)((p.C_out + T - 1) / T);
+    const size_t tiles = p.tiles_m * ((P_max + T - 1) / T);
+    hipLaunchKernelGGL((conv2d_small<T, WAVES>), dim3((unsigned)tiles, 1, classes), dim3(64 * WAVES), 0, ctx->stream, p);
+    return check_launch("conv2d_small");
+}
+
 }  // namespace
 
 bool conv_split_fits(const ConvSplitParams& p) {
@@ -295,6 +419,22 @@ size_t conv_split_tiles(const ConvSplitParams& p) {
     return s * s * (p.C_out <= 64 ? 1 : (p.C_out + 127) / 128) * ((pixels + 127) / 128);
 }
 
+// Fitted to 220 convolutions and gradients of up to 110 images' rows a side
+// (15 % rms): a wave's chain of K, a cost a tile, the operands a tile reads.
+// Beyond 20 us the fit is short of ragged and strided gathers.
+double conv_small_plan(const ConvSplitParams& p, int* tile) {
+    const size_t s = p.dgrad ? (size_t)p.stride : 1;
+    const double pixels = (double)p.N * (double)((p.Ho + s - 1) / s) * (double)((p.Wo + s - 1) / s);
+    const double taps = (double)((p.KH + s - 1) / s) * (double)((p.KW + s - 1) / s);
+    const double k_max = taps * p.C16, k = (double)p.KH * p.KW * p.C16 / (double)(s * s);
+    auto tiles = [&](double t) { return (double)(s * s) * std::ceil(p.C_out / t) * std::ceil(pixels / t); };
+    const double us16 = 1.5 + 2.9e-3 * k_max + tiles(16) * (3.1e-3 + 1.05e-5 * k);
+    const double us32 = 2.3 + 5.3e-3 * k_max + tiles(32) * (5.2e-3 + 2.05e-5 * k);
+    *tile = us16 <= us32 ? 16 : 32;
+    const double us = std::max(4.7, std::min(us16, us32));
+    return us + 0.7 * std::max(0.0, us - 20.0);
+}
+
 int launch_conv_split(lancius_hip_ctx* ctx, ConvSplitParams& p, const float* w) {
     if (w) {
         void* ws = nullptr;
@@ -305,6 +445,8 @@ int launch_conv_split(lancius_hip_ctx* ctx, ConvSplitParams& p, const float* w) 
     const size_t s = p.dgrad ? (size_t)p.stride : 1;
     const size_t pixels = (size_t)p.N * ((p.Ho + s - 1) / s) * ((p.Wo + s - 1) / s);
     const unsigned classes = (unsigned)(s * s);
+    if (p.small_tile == 32) return launch_small<32, 8>(ctx, p, pixels, classes);
+    if (p.small_tile == 16) return launch_small<16, 8>(ctx, p, pixels, classes);
     // 128 channels x 128 pixels, or 64 x 128 for at most 64 channels: four
     // waves, two workgroups a CU; grids of at most one tile a CU give each
     // tile eight waves in two k-groups

@@ -1357,7 +1357,8 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
     // (gemm_split.hip); both operands transposed, or one beyond 32-bit
     // offsets, stay with the fp32 kernels.
     if (!(ta && tb) && split_fits && (K >= 32 || big_tiles >= 768)) {
-        if (plan.tile >= 0) {
+        if (plan.tile >= 0 &&
+            (plan.splits == 1 || fixed || workspace_ready(ctx, count * plan.splits * M * N * sizeof(float)))) {
             const size_t steps = (K + 31) / 32, chunk = (steps + plan.splits - 1) / plan.splits;
             p.splits = (int)((steps + chunk - 1) / chunk);  // no empty K range
             p.kchunk = (int)(chunk * 32);

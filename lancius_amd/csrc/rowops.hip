@@ -873,7 +873,7 @@ int lancius_hip_cross_entropy_f32(lancius_hip_ctx* ctx, float* out, const float*
     // Up to 4096 rows need no scratch memory: a capture that has none yet
     // (it cannot allocate) records the one launch.
     const bool one = rows <= round * (cols <= 16 ? 4 : cols <= 256 ? 2 : 1) ||
-                     (rows <= 4096 && ctx->capturing && ctx->workspace_bytes < rows * sizeof(double));
+                     (rows <= 4096 && !workspace_ready(ctx, rows * sizeof(double)));
     void* ws = nullptr;
     if (!one)
         if (int rc = workspace(ctx, rows * sizeof(double), &ws)) return rc;
