@@ -8,7 +8,11 @@
 // Skipping key blocks that lie entirely above the diagonal is exactly the
 // reference's masking: exp(-1e9 - m) is 0 and the correction factor is 1.
 //
-// Fast kernel (D = 32, 64, 96, 128), "transposed" formulation so that every
+// More than 64 keys mostly run as split products (attention_split.hip); the
+// kernels here take short key ranges, small grids at D = 64, decode, and other
+// head dims.
+//
+// Matrix kernel (D = 32, 64, 96, 128), "transposed" formulation so that every
 // softmax statistic is lane-local:
 //   S^T[key][q] = K . Q^T    MFMA A = K tile (LDS), B = Q^T (registers)
 //   O^T[d][q]  += V^T . P^T  MFMA A = V^T (LDS),    B = P^T (the S^T registers)

@@ -7,6 +7,9 @@
 // ReLU on store (:168).  The reference has no bias; the device adds bias[co]
 // when one is given (NULL otherwise).
 //
+// This file: the entry points, the choice of kernel, and the fp32 kernels for
+// sizes between conv_split.hip's two and beyond 32-bit offsets.
+//
 // GEMM view: Out[co][P] = sum_k W[co][k] * X[k][P] with k = (ci, kh, kw) and
 // P = (n, ho, wo) running over every output pixel of the batch.  The OIHW
 // weight tensor already is the row-major [C_out][C_in*K_h*K_w] A operand.  The

@@ -3,7 +3,12 @@
 // (bleeding/v11A1/src/runtime/lancius_scheduler.c:222-234, which reads
 // M = a.shape[0], K = a.shape[1], N = b.shape[1]).
 //
-// Design:
+// This file: the dispatch (by what each kernel costs, gemm_plan and skinny_us),
+// the skinny kernel for few rows of a large B, and the fp32 kernels for sizes
+// between gemm_small.hip's and gemm_split.hip's, both operands transposed, and
+// operands beyond 32-bit offsets.
+//
+// Design of the staged fp32 kernel:
 //  * 256 threads = 4 wave64s arranged WGM x WGN; each wave owns a
 //    (BM/WGM) x (BN/WGN) block of C held in v_mfma_f32_32x32x2_f32
 //    accumulators (16 fp32 per lane per 32x32 sub-tile).

@@ -60,16 +60,6 @@ __device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// c + a . b over 16 k, smallest terms first.
-__device__ __forceinline__ f32x16 mfma_split(const SplitOperand& a, const SplitOperand& b, f32x16 c) {
-    c = mfma_bf16(a.l, b.h, c);
-    c = mfma_bf16(a.h, b.l, c);
-    c = mfma_bf16(a.m, b.m, c);
-    c = mfma_bf16(a.m, b.h, c);
-    c = mfma_bf16(a.h, b.m, c);
-    return mfma_bf16(a.h, b.h, c);
-}
-
 // An instruction that reads a matrix instruction's result needs wait states
 // that the compiler counts; across a branch it has been seen to count them
 // along the longer of two paths only (the reader got registers 14 and 15 of a
