@@ -1253,7 +1253,7 @@ double skinny_us(size_t count, size_t M, size_t K, size_t N, bool vb) {
     const double k = (double)K, bytes = 4.0 * (double)count * k * N;
     const double us = vb ? (M <= 16 ? (K <= 512 ? 4.9 : K <= 1664 && N <= 64 ? 5.8 : 6.3) : (K <= 512 ? 7.0 : 8.7))
                          : (M <= 16 ? 6.0 + std::min(5.0, 0.010 * k) : 8.0 + std::min(7.0, 0.014 * k));
-    return std::max(us, 3.0 + bytes / 4e6);
+    return std::max(us, 3.0 + bytes / 8e6);  // (8 x 1024 x 8192: 6.9; small tiles 12)
 }
 
 // fixed: when not null, split-K partials and arrival counters go to its
