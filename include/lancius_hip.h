@@ -369,8 +369,12 @@ LANCIUS_HIP_EXPORT int lancius_hip_stream_wait(lancius_hip_ctx* waiter, lancius_
 typedef struct lancius_hip_graph lancius_hip_graph;
 /* Record every launch enqueued on ctx between begin and end into a graph
  * instead of running it (ctx must own a stream: the null stream cannot be
- * captured).  Launches that allocate (first use of a workspace) must have
- * run once before capture. */
+ * captured).  Nothing can be allocated meanwhile: a call that needs more
+ * scratch memory than the context has by then is recorded with a kernel that
+ * needs none where there is one, and refused with -4 otherwise, so run the
+ * calls once before capture for the kernels that they have outside of it.
+ * The graph keeps the scratch memory that it recorded until it is destroyed:
+ * the context may grow more for later calls, or be destroyed first. */
 LANCIUS_HIP_EXPORT int lancius_hip_capture_begin(lancius_hip_ctx* ctx);
 LANCIUS_HIP_EXPORT int lancius_hip_capture_end(lancius_hip_ctx* ctx, lancius_hip_graph** out);
 LANCIUS_HIP_EXPORT int lancius_hip_graph_launch(lancius_hip_graph* graph, lancius_hip_ctx* ctx);

@@ -6,6 +6,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <mutex>
+#include <new>
 
 #include "common.hpp"
 
@@ -54,25 +55,60 @@ int cu_count(lancius_hip_ctx* ctx) {
     return ctx->cus;
 }
 
+namespace {
+
+// Gives up one hold on a block; the last one frees it (hipFree waits for the
+// device, so launches that still use it end first).
+void release(DeviceBlock* b) {
+    if (!b || b->holders.fetch_sub(1, std::memory_order_acq_rel) != 1) return;
+    int cur = -1;
+    const bool other = hipGetDevice(&cur) == hipSuccess && cur != b->device;
+    if (other) (void)hipSetDevice(b->device);
+    // (the thread may be recording on another context while it destroys a graph)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    (void)hipFree(b->ptr);
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (other) (void)hipSetDevice(cur);
+    delete b;
+}
+
+DeviceBlock* hold(DeviceBlock* b) {
+    b->holders.fetch_add(1, std::memory_order_relaxed);
+    return b;
+}
+
+// Replaces *slot by a block of `bytes`, whose first holder is the context.
+int grow(lancius_hip_ctx* ctx, DeviceBlock** slot, size_t bytes, const char* what) {
+    if (*slot) {
+        LANCIUS_HIP_TRY(hipStreamSynchronize(ctx->stream), what);
+        release(*slot);
+        *slot = nullptr;
+    }
+    void* p = nullptr;
+    LANCIUS_HIP_TRY(hipMalloc(&p, bytes), what);
+    DeviceBlock* b = new (std::nothrow) DeviceBlock{p, bytes, ctx->device, {1}};
+    if (!b) {
+        (void)hipFree(p);
+        return set_error(LANCIUS_HIP_ERR_OOM, "%s: host allocation failed", what);
+    }
+    *slot = b;
+    return 0;
+}
+
+}  // namespace
+
 int workspace(lancius_hip_ctx* ctx, size_t bytes, void** out) {
     *out = nullptr;
-    if (bytes <= ctx->workspace_bytes && ctx->workspace) {
-        *out = ctx->workspace;
-        return 0;
+    if (!ctx->workspace || bytes > ctx->workspace->bytes) {
+        LANCIUS_REQUIRE(!ctx->capturing, LANCIUS_HIP_ERR_UNSUPPORTED,
+                        "workspace of %zu bytes needed during graph capture: run the launches once before capturing",
+                        bytes);
+        const size_t want = (bytes + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
+        if (int rc = grow(ctx, &ctx->workspace, want, "workspace")) return rc;
     }
-    LANCIUS_REQUIRE(!ctx->capturing, LANCIUS_HIP_ERR_UNSUPPORTED,
-                    "workspace of %zu bytes needed during graph capture: run the launches once before capturing",
-                    bytes);
-    if (ctx->workspace) {
-        LANCIUS_HIP_TRY(hipStreamSynchronize(ctx->stream), "workspace sync");
-        LANCIUS_HIP_TRY(hipFree(ctx->workspace), "workspace free");
-        ctx->workspace = nullptr;
-        ctx->workspace_bytes = 0;
-    }
-    const size_t want = (bytes + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
-    LANCIUS_HIP_TRY(hipMalloc(&ctx->workspace, want), "workspace hipMalloc");
-    ctx->workspace_bytes = want;
-    *out = ctx->workspace;
+    ctx->recorded_workspace |= ctx->capturing;
+    *out = ctx->workspace->ptr;
     return 0;
 }
 
@@ -83,23 +119,19 @@ __global__ void zero_u32(unsigned* p, size_t n) {
 
 int counters(lancius_hip_ctx* ctx, size_t n, unsigned** out) {
     *out = nullptr;
-    if (n <= ctx->counters_n && ctx->counters) {
-        *out = ctx->counters;
-        return 0;
+    if (!ctx->counters || n * sizeof(unsigned) > ctx->counters->bytes) {
+        LANCIUS_REQUIRE(!ctx->capturing, LANCIUS_HIP_ERR_UNSUPPORTED, "counters needed during graph capture");
+        const size_t want = (n + 4095) & ~(size_t)4095;
+        if (int rc = grow(ctx, &ctx->counters, want * sizeof(unsigned), "counters")) return rc;
+        hipLaunchKernelGGL(zero_u32, dim3(64), dim3(256), 0, ctx->stream, (unsigned*)ctx->counters->ptr, want);
+        if (int rc = check_launch("zero_u32")) {
+            release(ctx->counters);
+            ctx->counters = nullptr;
+            return rc;
+        }
     }
-    LANCIUS_REQUIRE(!ctx->capturing, LANCIUS_HIP_ERR_UNSUPPORTED, "counters needed during graph capture");
-    if (ctx->counters) {
-        LANCIUS_HIP_TRY(hipStreamSynchronize(ctx->stream), "counters sync");
-        LANCIUS_HIP_TRY(hipFree(ctx->counters), "counters free");
-        ctx->counters = nullptr;
-        ctx->counters_n = 0;
-    }
-    const size_t want = (n + 4095) & ~(size_t)4095;
-    LANCIUS_HIP_TRY(hipMalloc((void**)&ctx->counters, want * sizeof(unsigned)), "counters hipMalloc");
-    hipLaunchKernelGGL(zero_u32, dim3(64), dim3(256), 0, ctx->stream, ctx->counters, want);
-    if (int rc = check_launch("zero_u32")) return rc;
-    ctx->counters_n = want;
-    *out = ctx->counters;
+    ctx->recorded_counters |= ctx->capturing;
+    *out = (unsigned*)ctx->counters->ptr;
     return 0;
 }
 
@@ -181,8 +213,8 @@ void lancius_hip_ctx_destroy(lancius_hip_ctx* ctx) {
     if (!ctx) return;
     (void)bind_device(ctx);
     (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->workspace) (void)hipFree(ctx->workspace);
-    if (ctx->counters) (void)hipFree(ctx->counters);
+    release(ctx->workspace);
+    release(ctx->counters);
     for (int s = 0; s < 3; ++s) {
         if (ctx->host_stage[s]) (void)hipHostFree(ctx->host_stage[s]);
         if (ctx->stage_done[s]) (void)hipEventDestroy(ctx->stage_done[s]);
@@ -215,6 +247,7 @@ int lancius_hip_capture_begin(lancius_hip_ctx* ctx) {
     if (int rc = bind_device(ctx)) return rc;
     LANCIUS_HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     ctx->capturing = 1;
+    ctx->recorded_workspace = ctx->recorded_counters = 0;
     return ok();
 }
 
@@ -237,6 +270,8 @@ int lancius_hip_capture_end(lancius_hip_ctx* ctx, lancius_hip_graph** out) {
         free(g);
         return from_hip(e, "hipGraphInstantiate");
     }
+    if (ctx->recorded_workspace) g->held[0] = hold(ctx->workspace);
+    if (ctx->recorded_counters) g->held[1] = hold(ctx->counters);
     *out = g;
     return ok();
 }
@@ -252,6 +287,7 @@ void lancius_hip_graph_destroy(lancius_hip_graph* graph) {
     if (!graph) return;
     (void)hipGraphExecDestroy(graph->exec);
     (void)hipGraphDestroy(graph->graph);
+    for (DeviceBlock* b : graph->held) release(b);
     free(graph);
 }
 

@@ -5,8 +5,13 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <atomic>
 
 #include "lancius_hip.h"
+
+namespace lancius {
+struct DeviceBlock;
+}
 
 struct lancius_hip_ctx {
     int device;
@@ -14,12 +19,12 @@ struct lancius_hip_ctx {
     hipEvent_t ev_start;
     hipEvent_t ev_stop;
     int timer_armed;
-    void* workspace;        // split-K partials, transposed conv weights
-    size_t workspace_bytes;
-    unsigned* counters;     // arrival counters of split reductions, kept at zero between calls
-    size_t counters_n;
+    lancius::DeviceBlock* workspace;  // split-K partials, transposed conv weights
+    lancius::DeviceBlock* counters;   // arrival counters of split reductions, kept at zero between calls
     int owns_stream;        // stream created by lancius_hip_ctx_create_own_stream
     int capturing;          // between lancius_hip_capture_begin and _end
+    int recorded_workspace; // the capture has recorded launches that use the workspace / the counters
+    int recorded_counters;
     hipEvent_t ev_order;    // lancius_hip_stream_wait
     void* host_stage[3];    // pinned staging of lancius_hip_upload_file, kept until destroy
     hipEvent_t stage_done[3];
@@ -29,9 +34,21 @@ struct lancius_hip_ctx {
 struct lancius_hip_graph {
     hipGraph_t graph;
     hipGraphExec_t exec;
+    lancius::DeviceBlock* held[2];  // the scratch memory its launches use
 };
 
 namespace lancius {
+
+// Scratch memory with its holders: the context that grew it, and every graph
+// recorded on that context whose launches hold its address.  Freed by the
+// last of them, so a context that needs more later, or is destroyed, leaves a
+// recorded graph's memory in place.
+struct DeviceBlock {
+    void* ptr;
+    size_t bytes;
+    int device;
+    std::atomic<int> holders;
+};
 
 // Records a failure in the thread-local status/message and returns the code.
 int set_error(int code, const char* fmt, ...);
@@ -46,15 +63,16 @@ int check_launch(const char* kernel);
 // Makes `ctx->device` current for the calling thread.
 int bind_device(lancius_hip_ctx* ctx);
 
-// Device scratch owned by the context, grown with hipMalloc on demand and
-// kept until the context is destroyed.  Calls on one context are ordered by
-// its stream, so one buffer serves every kernel of the context.
+// Device scratch of the context, grown with hipMalloc on demand and kept until
+// it is outgrown or the context destroyed, and by the graphs that recorded
+// it.  Calls on one context are ordered by its stream, so one buffer serves
+// every kernel of the context.
 int workspace(lancius_hip_ctx* ctx, size_t bytes, void** out);
 
 // Whether workspace(ctx, bytes) would succeed now: during a capture nothing can
 // be allocated, and a kernel that needs less scratch memory is taken instead.
 inline bool workspace_ready(const lancius_hip_ctx* ctx, size_t bytes) {
-    return !ctx->capturing || bytes == 0 || (ctx->workspace && bytes <= ctx->workspace_bytes);
+    return !ctx->capturing || bytes == 0 || (ctx->workspace && bytes <= ctx->workspace->bytes);
 }
 
 // Compute units of the context's device (cached in the context).
