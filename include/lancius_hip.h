@@ -450,6 +450,11 @@ LANCIUS_HIP_EXPORT int lancius_hip_upload_file(lancius_hip_ctx* ctx, const char*
  * Allocates and frees its own buffers; takes a few hundred milliseconds. */
 LANCIUS_HIP_EXPORT int lancius_hip_peak_probe(lancius_hip_ctx* ctx, int which, double* result);
 
+/* Name of the kernel that the calling thread launched last (back = 0), the one
+ * before it (1), ... up to 7; NULL where there is none.  A name has the tile
+ * and the other choices of the dispatch in it: which kernel a size gets. */
+LANCIUS_HIP_EXPORT const char* lancius_hip_last_kernel(int back);
+
 /* ---- reference-ABI bridge ------------------------------------------- */
 
 /* The fp32 matmul that the reference declares but never defines

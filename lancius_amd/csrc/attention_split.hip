@@ -412,7 +412,7 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
 template <int D, int KS>
 int launch(lancius_hip_ctx* ctx, const AttnParams& p, unsigned tasks) {
     hipLaunchKernelGGL((attention_split<D, KS>), dim3(tasks), dim3(256 * KS), 0, ctx->stream, p);
-    return check_launch("attention_split");
+    return check_launch(LANCIUS_KERNEL_NAME("attention_split D=%d x%d", D, KS));
 }
 
 }  // namespace

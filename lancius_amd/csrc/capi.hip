@@ -39,10 +39,23 @@ int from_hip(hipError_t e, const char* what) {
     return set_error(code, "%s: %s", what, hipGetErrorString(e));
 }
 
+// The calling thread's last launches, by name.
+constexpr unsigned kLaunchesKept = 8;
+static thread_local const char* t_launched[kLaunchesKept];
+static thread_local unsigned t_launches = 0;
+
 int check_launch(const char* kernel) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return from_hip(e, kernel);
+    t_launched[t_launches++ % kLaunchesKept] = kernel;
     return 0;
+}
+
+KernelName::KernelName(const char* fmt, ...) {
+    va_list ap;
+    va_start(ap, fmt);
+    vsnprintf(text, sizeof(text), fmt, ap);
+    va_end(ap);
 }
 
 int cu_count(lancius_hip_ctx* ctx) {
@@ -153,6 +166,11 @@ extern "C" {
 
 const char* lancius_hip_last_error(void) { return t_message; }
 int lancius_hip_last_status(void) { return t_status; }
+
+const char* lancius_hip_last_kernel(int back) {
+    if (back < 0 || (unsigned)back >= kLaunchesKept) return nullptr;
+    return t_launched[(t_launches - 1 - (unsigned)back) % kLaunchesKept];
+}
 
 int lancius_hip_device_count(void) {
     int n = 0;

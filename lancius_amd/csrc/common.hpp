@@ -57,8 +57,21 @@ int ok();
 // Maps a HIP error to a status (OOM -> -1, everything else -> -10).
 int from_hip(hipError_t e, const char* what);
 
-// Checks a kernel launch: reads hipGetLastError() after <<<>>>.
+// Checks a kernel launch (hipGetLastError() after <<<>>>) and notes its name
+// for lancius_hip_last_kernel; `kernel` stays valid.
 int check_launch(const char* kernel);
+
+// The name of a launch with the template arguments of the launching function:
+// formatted once per instantiation.
+struct KernelName {
+    char text[64];
+    __attribute__((format(printf, 2, 3))) explicit KernelName(const char* fmt, ...);
+};
+#define LANCIUS_KERNEL_NAME(...)                       \
+    ([] {                                              \
+        static const ::lancius::KernelName n(__VA_ARGS__); \
+        return n.text;                                 \
+    }())
 
 // Makes `ctx->device` current for the calling thread.
 int bind_device(lancius_hip_ctx* ctx);

@@ -1156,18 +1156,20 @@ int launch(lancius_hip_ctx* ctx, ConvParams& p) {
         if (p.sk_wgs > 0)
             if (int rc = counters(ctx, grid - (size_t)p.sk_dp, &p.sk_ctr)) return rc;
         hipLaunchKernelGGL(kern, dim3((unsigned)(p.sk_dp + p.sk_wgs)), dim3(kThreads), 0, ctx->stream, p);
-        return check_launch("conv2d_direct");
+        return check_launch(p.sk_wgs == 0  ? LANCIUS_KERNEL_NAME("conv2d_direct %dx%d", BM, BN)
+                            : p.sk_dp == 0 ? LANCIUS_KERNEL_NAME("conv2d_direct %dx%d all shared", BM, BN)
+                                           : LANCIUS_KERNEL_NAME("conv2d_direct %dx%d tail shared", BM, BN));
     }
     if constexpr (BM == 32) {
         if (wt_layout) {
             hipLaunchKernelGGL((conv2d_implicit_gemm<BM, BN, 16, WGM, WGN, KH_T, KW_T, true>), dim3((unsigned)grid),
                                dim3(kThreads), 0, ctx->stream, p);
-            return check_launch("conv2d_implicit_gemm");
+            return check_launch("conv2d_implicit_gemm 32x128 per channel");
         }
     }
     hipLaunchKernelGGL((conv2d_implicit_gemm<BM, BN, 16, WGM, WGN, KH_T, KW_T, false>), dim3((unsigned)grid),
                        dim3(kThreads), 0, ctx->stream, p);
-    return check_launch("conv2d_implicit_gemm");
+    return check_launch(LANCIUS_KERNEL_NAME("conv2d_implicit_gemm %dx%d", BM, BN));
 }
 
 int default_tile(size_t C_out) { return C_out > 64 ? 1 : C_out > 32 ? 2 : 3; }
@@ -1531,7 +1533,7 @@ extern "C" int lancius_hip_conv2d_bwd_weight_f32(lancius_hip_ctx* ctx, float* dw
         hipLaunchKernelGGL((conv2d_wgrad_mfma<128, 64, bk>), grid, dim3(256), 0, ctx->stream, p);
     else
         hipLaunchKernelGGL((conv2d_wgrad_mfma<64, 64, bk>), grid, dim3(256), 0, ctx->stream, p);
-    if (int rc = check_launch("conv2d_wgrad_mfma")) return rc;
+    if (int rc = check_launch(direct ? "conv2d_wgrad_direct" : "conv2d_wgrad_mfma")) return rc;
     if (p.splits > 1)
         if (int rc = launch_wgrad_reduce(ctx, dw, p.ws, C_out * J, p.splits)) return rc;
     return ok();

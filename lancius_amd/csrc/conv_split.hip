@@ -370,7 +370,7 @@ int launch(lancius_hip_ctx* ctx, ConvSplitParams& p, size_t P_max, unsigned clas
     const size_t tiles = p.tiles_m * ((P_max + BN - 1) / BN);
     hipLaunchKernelGGL((conv2d_split<BM, BN, WM, WN, KG>), dim3((unsigned)tiles, 1, classes),
                        dim3(64 * (BM / WM) * (BN / WN) * KG), 0, ctx->stream, p);
-    return check_launch("conv2d_split");
+    return check_launch(LANCIUS_KERNEL_NAME("conv2d_split %dx%d x%d", BM, BN, KG));
 }
 
 template <int T, int WAVES>
@@ -378,7 +378,7 @@ int launch_small(lancius_hip_ctx* ctx, ConvSplitParams& p, size_t P_max, unsigne
     p.tiles_m = (uint32_t)((p.C_out + T - 1) / T);
     const size_t tiles = p.tiles_m * ((P_max + T - 1) / T);
     hipLaunchKernelGGL((conv2d_small<T, WAVES>), dim3((unsigned)tiles, 1, classes), dim3(64 * WAVES), 0, ctx->stream, p);
-    return check_launch("conv2d_small");
+    return check_launch(LANCIUS_KERNEL_NAME("conv2d_small %dx%d", T, T));
 }
 
 }  // namespace

@@ -1007,8 +1007,11 @@ int launch_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec) {
                     "gemm: configuration %dx%d/%d without this variant (split %d, vec %d)", BM, BN, BK, (int)split,
                     (int)vec);
     const dim3 block(kThreads * KG);
+#define NAME(what) LANCIUS_KERNEL_NAME("gemm_f32_mfma %dx%d/%d x%d %c%c " what, BM, BN, BK, KG, TA ? 'T' : 'N', TB ? 'T' : 'N')
+    const char* name = nullptr;
     if constexpr (SPLITS && VECS) {
         if (vec && split) {
+            name = NAME("float4 split K");
             hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, BK, WGM, WGN, true, true, SOCC, TA, TB, KG>), grid, block, 0,
                                ctx->stream, p);
             goto launched;
@@ -1016,6 +1019,7 @@ int launch_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec) {
     }
     if constexpr (VECS) {
         if (vec) {
+            name = NAME("float4");
             hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, BK, WGM, WGN, true, false, OCC, TA, TB, KG>), grid, block, 0,
                                ctx->stream, p);
             goto launched;
@@ -1023,15 +1027,18 @@ int launch_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec) {
     }
     if constexpr (SPLITS) {
         if (split) {
+            name = NAME("scalar split K");
             hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, BK, WGM, WGN, false, true, SOCC, TA, TB, KG>), grid, block, 0,
                                ctx->stream, p);
             goto launched;
         }
     }
+    name = NAME("scalar");
     hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, BK, WGM, WGN, false, false, SOCC, TA, TB, KG>), grid, block, 0,
                        ctx->stream, p);
 launched:
-    if (int rc = check_launch("gemm_f32_mfma")) return rc;
+#undef NAME
+    if (int rc = check_launch(name)) return rc;
     return split ? launch_splitk_reduce(ctx, p, count) : 0;
 }
 
@@ -1441,7 +1448,7 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
         const int kg = t64 <= 384 ? 4 : 2;
         hipLaunchKernelGGL((kg == 2 ? gemm_f32_direct_kg<2> : gemm_f32_direct_kg<4>),
                            dim3(p.tiles_m * p.tiles_n, 1, (unsigned)count), dim3(256 * kg), 0, ctx->stream, p);
-        if (int rc = check_launch("gemm_f32_direct_kg")) return rc;
+        if (int rc = check_launch(kg == 2 ? "gemm_f32_direct_kg x2" : "gemm_f32_direct_kg x4")) return rc;
         return ok();
     }
     if (splits > 1) {

@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_f32_small(const GemmParams p)
 }
 
 template <int T, int WAVES>
-void launch(hipStream_t stream, GemmParams& p, int count, bool ta, bool tb) {
+int launch(hipStream_t stream, GemmParams& p, int count, bool ta, bool tb) {
     p.tiles_m = (uint32_t)((p.M + T - 1) / T);
     p.tiles_n = (uint32_t)((p.N + T - 1) / T);
     const dim3 grid(p.tiles_m * p.tiles_n, 1, (unsigned)count), block(64 * WAVES);
@@ -142,6 +142,7 @@ void launch(hipStream_t stream, GemmParams& p, int count, bool ta, bool tb) {
         hipLaunchKernelGGL((gemm_f32_small<T, false, true, WAVES>), grid, block, 0, stream, p);
     else
         hipLaunchKernelGGL((gemm_f32_small<T, false, false, WAVES>), grid, block, 0, stream, p);
+    return check_launch(LANCIUS_KERNEL_NAME("gemm_f32_small %dx%d x%d", T, T, WAVES));
 }
 
 }  // namespace
@@ -167,15 +168,8 @@ SmallPlan gemm_small_plan(size_t count, size_t M, size_t K, size_t N, bool tb) {
 
 int launch_gemm_small(lancius_hip_ctx* ctx, GemmParams& p, int count, bool ta, bool tb, int tile) {
     // 16 waves at a long K are for the sums: chains no longer than before
-    if (tile == 32 && p.K < 512)
-        launch<32, 8>(ctx->stream, p, count, ta, tb);
-    else if (tile == 32)
-        launch<32, 16>(ctx->stream, p, count, ta, tb);
-    else if (p.K < 1024)
-        launch<16, 8>(ctx->stream, p, count, ta, tb);
-    else
-        launch<16, 16>(ctx->stream, p, count, ta, tb);
-    return check_launch("gemm_f32_small");
+    if (tile == 32) return p.K < 512 ? launch<32, 8>(ctx->stream, p, count, ta, tb) : launch<32, 16>(ctx->stream, p, count, ta, tb);
+    return p.K < 1024 ? launch<16, 8>(ctx->stream, p, count, ta, tb) : launch<16, 16>(ctx->stream, p, count, ta, tb);
 }
 
 }  // namespace lancius

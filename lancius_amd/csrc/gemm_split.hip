@@ -135,15 +135,20 @@ void launch(hipStream_t stream, GemmParams& p, int count, bool ta, bool tb) {
 }  // namespace
 
 int launch_gemm_split(lancius_hip_ctx* ctx, GemmParams& p, int count, bool ta, bool tb, int tile) {
-    if (tile == kSplit256)
+    const char* name = "gemm_f32_split 128x128";
+    if (tile == kSplit256) {
+        name = "gemm_f32_split 256x256";
         launch<256, 256, 64, 128, 1, false, kOneSum, 5>(ctx->stream, p, count, ta, tb);
-    else if (tile == kSplit256x128)
+    } else if (tile == kSplit256x128) {
+        name = "gemm_f32_split 256x128";
         launch<256, 128, 64, 64, 1, false, kTwoSums, 0>(ctx->stream, p, count, ta, tb);
-    else if (p.splits == 1)
+    } else if (p.splits == 1) {
         launch<128, 128, 64, 64, 2, false, kTwoSums, 4>(ctx->stream, p, count, ta, tb);
-    else
+    } else {
+        name = "gemm_f32_split 128x128 split K";
         launch<128, 128, 64, 64, 2, true, kTwoSums, 4>(ctx->stream, p, count, ta, tb);
-    return check_launch("gemm_f32_split");
+    }
+    return check_launch(name);
 }
 
 }  // namespace lancius

@@ -279,7 +279,7 @@ int launch_wgrad_split(lancius_hip_ctx* ctx, WgradSplitParams& p) {
         launch<128, 128, 64, 64, 2>(ctx->stream, p);
     else
         launch<64, 128, 64, 32, 2>(ctx->stream, p);
-    return check_launch("wgrad_split");
+    return check_launch(p.C_out > 64 ? "wgrad_split 128x128" : "wgrad_split 64x128");
 }
 
 }  // namespace lancius

@@ -126,6 +126,8 @@ def _declare_hip(lib: C.CDLL) -> C.CDLL:
     lib.lancius_hip_ctx_stream.argtypes = [vp]
     lib.lancius_hip_ctx_stream.restype = vp
     lib.lancius_hip_stream_wait.argtypes = [vp, vp]
+    lib.lancius_hip_last_kernel.argtypes = [C.c_int]
+    lib.lancius_hip_last_kernel.restype = C.c_char_p
     lib.lancius_hip_capture_begin.argtypes = [vp]
     lib.lancius_hip_capture_end.argtypes = [vp, C.POINTER(vp)]
     lib.lancius_hip_graph_launch.argtypes = [vp, vp]
@@ -245,6 +247,11 @@ class Device:
         _check(self.lib.lancius_hip_download(self.ctx, out.ctypes.data_as(C.c_void_p), C.c_void_p(int(src)),
                                              out.nbytes))
         return out
+
+    def launched(self, n: int = 1) -> list[str]:
+        """Names of the calling thread's last n (at most 8) kernel launches, the newest first."""
+        names = [self.lib.lancius_hip_last_kernel(i) for i in range(n)]
+        return [s.decode() for s in names if s]
 
     def synchronize(self) -> None:
         _check(self.lib.lancius_hip_synchronize(self.ctx))

@@ -17,6 +17,7 @@ def _run(dev, A, B, M, K, N, ta=False, tb=False, bias=None, act=ACT_NONE, residu
     db = dev.upload(bias) if bias is not None else None
     dR = dev.upload(residual) if residual is not None else None
     dev.gemm_ex(dC, dA, dB, M, K, N, trans_a=ta, trans_b=tb, bias=db, act=act, residual=dR)
+    _run.kernels = dev.launched(2)
     got = dev.download(dC, (M * N + 1024,))
     assert (got[M * N:] == 7.0).all()  # nothing is stored past C
     for b in (dA, dB, dC, db, dR):
@@ -34,7 +35,8 @@ SHAPES = [
     (1537, 300, 2999, "256x128, ragged"),
     (2048, 257, 3071, "256x128, one k over"),
     (1024, 304, 4096, "128x128"),
-    (1031, 289, 4093, "128x128, ragged"),
+    (1031, 289, 4093, "256x128, seven rows over"),
+    (1153, 289, 2303, "128x128, ragged"),
     (641, 3203, 383, "128x128, split K, ragged"),
     (512, 4096, 512, "128x128, split K"),
 ]
@@ -51,6 +53,8 @@ def test_gemm_split_shapes(dev, M, K, N, what, layout):
     R = prng.normal(6, (M, N)) if layout != "NT" else None
     got = _run(dev, np.ascontiguousarray(A.T) if ta else A, np.ascontiguousarray(B.T) if tb else B, M, K, N, ta, tb,
                bias, act, R)
+    assert "gemm_f32_split " + what.split(", ")[0] in _run.kernels[0 if "split K" not in what else 1]
+    assert ("split K" in what) == (_run.kernels[0] == "splitk_reduce")
     ref = A.astype(np.float64) @ B.astype(np.float64)
     if bias is not None:
         ref = ref + bias.astype(np.float64)
