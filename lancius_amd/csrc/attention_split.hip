@@ -13,6 +13,13 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kQueries = 128;  // per workgroup, 32 per wave
 constexpr int kKeys = 32;      // per step
 
+// The scaled range (split.hpp) here: V is scaled as there.  Q (times the score
+// scale) carries 2^32: past 2^96 it overflows and is recomputed, so what a key
+// below 2^-110 loses, 2^-134, stays under 2^-31 in a score, whose absolute
+// error counts, and K needs no scale.  Nor have probabilities one: below
+// 2^-110 they keep 8 to 16 bits, an error of 2^-134 of the largest.
+constexpr float kQueryUp = 0x1p32f;
+
 // D = head dim; KS = 2: eight waves, the second four taking the odd key
 // blocks of the same queries (grids of at most one tile per CU).
 //
@@ -102,7 +109,7 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
         for (int s = 0; s < QS; ++s) {
             const f32x4 x = src[4 * s], y = src[4 * s + 1];
             f32x8 v = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
-            v = v * p.qscale;
+            v = v * (p.qscale * kQueryUp);
             qf[s] = split8(v);
             // (this lane's own slot: with two k-groups both write the same values)
             if constexpr (QL) *(bf16x8*)(ql + s * 1024) = qf[s].l;
@@ -159,10 +166,10 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
             }
         }
     };
-    auto store_block = [&](char* to) {
+    auto store_block = [&](auto role, char* to) {
 #pragma unroll
         for (int c = 0; c < NB; ++c) {
-            const SplitOperand s = split8(sreg[c]);
+            const SplitOperand s = decltype(role)::value ? split8(sreg[c]) : split8_up(sreg[c]);
             char* at = to + s_wr + c * 512;
             *(bf16x8*)at = s.h;
             *(bf16x8*)(at + PART) = s.m;
@@ -191,22 +198,22 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
             for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) > lim ? -INFINITY : s[r];
         }
     };
-    // Running maximum and sum; probabilities in place of the scores.  Returns
-    // the factor of the sums so far.
-    auto softmax = [&](f32x16& s) {
+    // Running maximum and sum; probabilities in place of the scores, which come
+    // multiplied by 1 / down.  Returns the factor of the sums so far.
+    auto softmax = [&](f32x16& s, float down) {
         float mx = s[0];
 #pragma unroll
         for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
         const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx),
                                                          false, false);  // the other half's maximum
         mx = fmaxf(__builtin_bit_cast(float, (unsigned)sw[0]), __builtin_bit_cast(float, (unsigned)sw[1]));
-        const float m_new = fmaxf(m_run, mx);
+        const float m_new = fmaxf(m_run, mx * down);
         const float corr = exp2_raw(m_run - m_new);
         m_run = m_new;
         float psum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            s[r] = exp2_raw(s[r] - m_new);
+            s[r] = exp2_raw(fmaf(s[r], down, -m_new));
             psum += s[r];
         }
         l_part = l_part * corr + psum;
@@ -245,7 +252,7 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
         f32x16 s_cur = {};
         load_block(role, grp);
         if (IS_K) {
-            store_block(kbase);
+            store_block(role, kbase);
             load_block(role, grp + KS);
         }
         __syncthreads();
@@ -254,7 +261,7 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
             mask(s_cur, grp * kKeys);
             __syncthreads();
             if (IS_K) {
-                store_block(kbase);
+                store_block(role, kbase);
                 load_block(role, grp + 2 * KS);
             }
             __syncthreads();
@@ -272,7 +279,7 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
                     s_cur = scores();
                     mask(s_cur, kb);
                 }
-                corr = softmax(s_cur);
+                corr = softmax(s_cur, 1.0f / kQueryUp);
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
                     f32x8 x;
@@ -282,12 +289,12 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
                 }
             }
             if (!IS_K) {  // every wave is past the last step's V
-                store_block(vbase);
+                store_block(role, vbase);
                 load_block(role, blk + KS);
             }
             __syncthreads();
             if (IS_K) {  // every wave is past the staged K
-                store_block(kbase);
+                store_block(role, kbase);
                 load_block(role, blk + (PIPE ? 3 : 2) * KS);
             }
             if (active) {
@@ -327,15 +334,19 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
             key_loop(std::integral_constant<bool, false>{});
     }
 
-    // Sums that are not all finite (infinite or NaN inputs, values above the
-    // largest bf16): the wave's key blocks again with the fp32 instructions.
+    // Sums that are not all finite (infinite or NaN inputs, values or scores
+    // beyond the scaled range): the wave's key blocks again with the fp32
+    // instructions.
     float none = 0.0f, probe = l_part * 0.0f;
     asm("" : "+v"(none));
 #pragma unroll
     for (int e = 0; e < NB; ++e)
 #pragma unroll
         for (int r = 0; r < 16; ++r) probe = fmaf(o_acc[e][r], none, probe);
-    if (__any(!(probe == 0.0f))) {
+    if (!__any(!(probe == 0.0f))) {
+#pragma unroll
+        for (int e = 0; e < NB; ++e) o_acc[e] *= 1.0f / kSplitUp;
+    } else {
 #pragma unroll
         for (int e = 0; e < NB; ++e) o_acc[e] = f32x16{};
         m_run = -1e30f;
@@ -355,7 +366,7 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
             }
             settle(s_acc);
             mask(s_acc, kb);
-            const float corr = softmax(s_acc);
+            const float corr = softmax(s_acc, 1.0f);
 #pragma unroll
             for (int e = 0; e < NB; ++e)
 #pragma unroll

@@ -98,7 +98,7 @@ struct PixelLoader {
 
 template <int BM, int BN, int WM, int WN, int KG>
 __global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, 2) conv2d_split(const ConvSplitParams p) {
-    using T = SplitTile<BM, BN, WM, WN, KG, kTwoSums, 0>;
+    using T = SplitTile<BM, BN, WM, WN, KG, kTwoSums, 3>;
     constexpr int TN = T::TN;
     static_assert(T::CB == 2, "a thread stages both k halves of a pixel");
     __shared__ __attribute__((aligned(16))) char smem[T::SMEM];

@@ -143,10 +143,10 @@ int launch_gemm_split(lancius_hip_ctx* ctx, GemmParams& p, int count, bool ta, b
         name = "gemm_f32_split 256x128";
         launch<256, 128, 64, 64, 1, false, kTwoSums, 0>(ctx->stream, p, count, ta, tb);
     } else if (p.splits == 1) {
-        launch<128, 128, 64, 64, 2, false, kTwoSums, 4>(ctx->stream, p, count, ta, tb);
+        launch<128, 128, 64, 64, 2, false, kTwoSums, 5>(ctx->stream, p, count, ta, tb);
     } else {
         name = "gemm_f32_split 128x128 split K";
-        launch<128, 128, 64, 64, 2, true, kTwoSums, 4>(ctx->stream, p, count, ta, tb);
+        launch<128, 128, 64, 64, 2, true, kTwoSums, 5>(ctx->stream, p, count, ta, tb);
     }
     return check_launch(name);
 }

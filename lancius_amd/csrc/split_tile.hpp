@@ -98,7 +98,7 @@ struct SplitTile {
         const int b_rd = A_BYTES + (lk * BN + wn * WN + lr) * 16;
         auto stage = [&](int buf, int c) {
             if (c >= CN) return;
-            const SplitOperand s = split8(ld.chunk(c));
+            const SplitOperand s = split8_up(ld.chunk(c));
             char* const at = base + buf + (IS_A ? 0 : A_BYTES) + ld.wr[c < CN ? c : 0];
             *(bf16x8*)(at) = s.h;
             *(bf16x8*)(at + PL) = s.m;
@@ -163,7 +163,7 @@ struct SplitTile {
         }
     }
 
-    // The whole sums, after run() and a settle.  Two k-groups: each keeps half
+    // The whole sums, after run() and a settle, as the operands have them.  Two k-groups: each keeps half
     // of the wave's block rows (acc[0 .. TS), rows wm WM + 32 grp ..) and adds
     // the other group's sums of them (a + b is the same either way round, so
     // results do not depend on which group ends first).
@@ -176,6 +176,10 @@ struct SplitTile {
 #pragma unroll
                 for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
         }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] *= kSplitDown;
         if constexpr (KG > 1) {
             float* const red = (float*)smem;
             auto at = [&](int from, int j, int r) { return ((from * GW + gw) * TN + j) * 1024 + r * 64 + lane; };
@@ -195,9 +199,8 @@ struct SplitTile {
     // the wave's first block row of those it keeps
     __device__ __forceinline__ int row0() const { return wm * WM + 32 * (KG > 1 ? grp : 0); }
 
-    // Some kept sum is not finite (an infinite or NaN input, a value above the
-    // largest bf16, or a product that overflows): the wave recomputes its
-    // blocks in fp32.
+    // Some kept sum is not finite (an infinite or NaN input, or a value or
+    // product beyond the scaled range): the wave recomputes its blocks in fp32.
     __device__ __forceinline__ bool not_finite() const {
         float none = 0.0f, probe = 0.0f;
         asm("" : "+v"(none));  // a register: the compiler may not fold x * 0

@@ -45,6 +45,24 @@ def top2_margin(logits) -> float:
     return float(np.min(top[:, 1] - top[:, 0]))
 
 
+def two_norm_error(y, ref) -> float:
+    """Norm of the error over the norm of the result, in 64 bits."""
+    import numpy as np
+
+    y, ref = np.asarray(y, dtype=np.float64).ravel(), np.asarray(ref, dtype=np.float64).ravel()
+    scale = np.abs(ref).max()  # (squares of results near the ends of fp32's range)
+    return float(np.linalg.norm((y - ref) / scale) / np.linalg.norm(ref / scale))
+
+
+def fp32_sum_error(k: int) -> float:
+    """What the two-norm error of sums of k random fp32 products stays under
+    when they are added in one chain: addition i rounds by at most 2^-24 of a
+    partial sum that has grown to sqrt(i / k) of the result, uniformly, so the
+    errors add up to 2^-24 sqrt(k / 6) (0.41 sqrt(k)); the products' own
+    rounding and a last one on top."""
+    return 2.0 ** -24 * (1.0 + 0.5 * k ** 0.5)
+
+
 def record_parity(config: str, err: float, bound: float, **extra) -> None:
     """Print one parity measurement (normwise error against its bound and
     any extra fields, e.g. top-2 margins) and, when the environment variable

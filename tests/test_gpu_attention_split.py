@@ -6,7 +6,7 @@ import pytest
 
 import oracle
 from lancius_amd import prng
-from tests.conftest import case
+from tests.conftest import case, fp32_sum_error, two_norm_error
 
 pytestmark = pytest.mark.gpu
 
@@ -17,6 +17,7 @@ def _run(dev, q, k, v, causal):
     dq, dk, dv, do = dev.upload(q), dev.upload(k), dev.upload(v), dev.alloc(q.nbytes + 1024)
     dev.fill(do, 7.0, q.size + 256)
     dev.attention_gqa(do, dq, dk, dv, B, Sq, Skv, Hq, Hkv, D, causal)
+    _run.kernel = dev.launched()[0]
     got = dev.download(do, (q.size + 256,))
     assert (got[q.size:] == 7.0).all()  # nothing is stored past the output
     for b in (dq, dk, dv, do):
@@ -95,3 +96,20 @@ def test_attention_split_non_finite(dev, D, causal):
         scale = 2.0 ** -100 if (part & big).any() else 1.0
         err = oracle.normwise_error(np.where(part, got, 0.0).astype(np.float64) * scale, np.where(part, ref, 0.0) * scale)
         assert err <= oracle.tolerance(Skv)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("q_exp,k_exp,v_exp", [(0, 0, 0), (0, 0, -118), (0, 0, 100), (-118, 118, 0), (118, -118, 0), (90, -90, -100)])
+def test_attention_split_range(dev, q_exp, k_exp, v_exp, D, causal):
+    """Operands at the ends of fp32's range whose scores are ordinary: each
+    keeps its 24 bits.  A score rounds as a sum over D, and its probability by
+    that times its size (at most 4 or so)."""
+    shape = (9, 130, 150, 16, 16)
+    case(f"attention split range D={D} causal={causal} 2^{q_exp} 2^{k_exp} 2^{v_exp}")
+    q, k, v = _inputs(4100 + D, *shape, D)
+    two = np.float32(2.0)
+    q, k, v = q * two ** np.float32(q_exp), k * two ** np.float32(k_exp), v * two ** np.float32(v_exp)
+    got = _run(dev, q, k, v, causal)
+    assert "attention_split" in _run.kernel, _run.kernel
+    assert two_norm_error(got, _ref(q, k, v, causal)) <= fp32_sum_error(shape[2]) + 4 * fp32_sum_error(D)

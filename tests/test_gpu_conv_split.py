@@ -8,7 +8,7 @@ import torch.nn.functional as F
 
 import oracle
 from lancius_amd import ACT_NONE, ACT_RELU, prng
-from tests.conftest import case
+from tests.conftest import case, fp32_sum_error, two_norm_error
 
 pytestmark = pytest.mark.gpu
 
@@ -29,9 +29,11 @@ def _forward(dev, x, w, bias, stride, pad, act, packed):
         pk = dev.alloc(dev.conv2d_packed_bytes(C_out, C_in, KH, KW))
         dev.conv2d_pack_weight(pk, dw, C_out, C_in, KH, KW)
         dev.conv2d_packed(do, dx, pk, db, N, C_in, H, W, C_out, KH, KW, stride, pad, act)
+        _forward.kernel = dev.launched()[0]
         pk.free()
     else:
         dev.conv2d(do, dx, dw, db, N, C_in, H, W, C_out, KH, KW, stride, pad, act)
+        _forward.kernel = dev.launched()[0]
     got = dev.download(do, (n + 1024,))
     assert (got[n:] == 7.0).all()  # nothing is stored past the output
     for b in (dx, dw, do, db):
@@ -47,6 +49,7 @@ def _bwd_input(dev, dy, w, H, W, stride, pad):
     dg, dw, do = dev.upload(dy), dev.upload(w), dev.alloc(4 * n + 4096)
     dev.fill(do, 7.0, n + 1024)
     dev.conv2d_bwd_input(do, dg, dw, N, C_in, H, W, C_out, Ho, Wo, KH, KW, stride, pad)
+    _bwd_input.kernel = dev.launched()[0]
     got = dev.download(do, (n + 1024,))
     assert (got[n:] == 7.0).all()
     for b in (dg, dw, do):
@@ -123,3 +126,28 @@ def test_conv_split_non_finite(dev, stride):
     for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
         err = oracle.normwise_error(np.where(part, got, 0).astype(np.float64) * scale, np.where(part, ref, 0) * scale)
         assert err <= oracle.tolerance(C_in * 9)
+
+
+@pytest.mark.parametrize("exponent", [0, -118, -126, -140])
+@pytest.mark.parametrize("what", ["forward", "gradient", "gradient, stride 2"])
+def test_conv_split_small_operands(dev, what, exponent):
+    """The image (or dY), then the filter, at the low end of fp32's range, the
+    other large enough for ordinary results: all 24 bits count there too."""
+    case(f"conv split small operands {what} 2^{exponent}")
+    N, C_in, H, W, C_out = 16, 64, 56, 56, 128
+    stride = 2 if "stride" in what else 1
+    Ho, Wo = _out(H, 3, stride, 1), _out(W, 3, stride, 1)
+    for small in ("image", "filter"):
+        w = prng.normal(6301, (C_out, C_in, 3, 3))
+        x = prng.normal(6300, (N, C_in, H, W) if what == "forward" else (N, C_out, Ho, Wo))
+        up, down = np.float32(2.0 ** (-exponent // 3)), np.float32(2.0) ** np.float32(exponent)
+        x, w = (x * down, w * up) if small == "image" else (x * up, w * down)
+        x64, w64 = torch.from_numpy(x).double(), torch.from_numpy(w).double()
+        if what == "forward":
+            got, kernel = _forward(dev, x, w, None, 1, 1, ACT_NONE, True), _forward.kernel
+            ref = F.conv2d(x64, w64, None, 1, 1)
+        else:
+            got, kernel = _bwd_input(dev, x, w, H, W, stride, 1), _bwd_input.kernel
+            ref = F.conv_transpose2d(x64, w64, None, stride, 1, output_padding=stride - 1)
+        assert "conv2d_split" in kernel, kernel
+        assert two_norm_error(got, ref.numpy()) <= fp32_sum_error(9 * (C_in if what == "forward" else C_out)), small

@@ -6,7 +6,7 @@ import pytest
 
 import oracle
 from lancius_amd import ACT_GELU, ACT_NONE, ACT_RELU, prng
-from tests.conftest import case
+from tests.conftest import case, fp32_sum_error, two_norm_error
 
 pytestmark = pytest.mark.gpu
 
@@ -85,6 +85,23 @@ def test_gemm_split_range(dev, layout, exponent):
     got = _run(dev, np.ascontiguousarray(A.T) if ta else A, np.ascontiguousarray(B.T) if tb else B, M, K, N, ta, tb)
     ref = A.astype(np.float64) @ B.astype(np.float64)
     assert oracle.normwise_error(got, ref) <= oracle.tolerance(K)
+
+
+@pytest.mark.parametrize("layout", ["NN", "TN", "NT"])
+@pytest.mark.parametrize("exponent", [0, -115, -120, -126, -140])
+@pytest.mark.parametrize("M,K,N", [(1031, 289, 4093), (3456, 64, 3712), (512, 4096, 512)])
+def test_gemm_split_small_operands(dev, M, K, N, exponent, layout):
+    """One operand at the low end of fp32's range, subnormals included, with
+    the other large enough for ordinary results: all 24 bits count there too."""
+    case(f"gemm split small operands {layout} {M}x{K}x{N} 2^{exponent}")
+    ta, tb = layout[0] == "T", layout[1] == "T"
+    for small in "AB":
+        A, B = prng.normal(13, (M, K)), prng.normal(14, (K, N))
+        up, down = np.float32(2.0 ** (-exponent // 3)), np.float32(2.0) ** np.float32(exponent)
+        A, B = (A * down, B * up) if small == "A" else (A * up, B * down)
+        got = _run(dev, np.ascontiguousarray(A.T) if ta else A, np.ascontiguousarray(B.T) if tb else B, M, K, N, ta, tb)
+        assert any("gemm_f32_split" in k for k in _run.kernels)
+        assert two_norm_error(got, A.astype(np.float64) @ B.astype(np.float64)) <= fp32_sum_error(K), small
 
 
 @pytest.mark.parametrize("layout", ["NN", "TN", "NT"])

@@ -8,7 +8,7 @@ import torch.nn.functional as F
 
 import oracle
 from lancius_amd import prng
-from tests.conftest import case
+from tests.conftest import case, fp32_sum_error, two_norm_error
 
 pytestmark = pytest.mark.gpu
 
@@ -20,6 +20,7 @@ def _run(dev, x, dy, KH, KW, stride, pad):
     dx, dg, do = dev.upload(x), dev.upload(dy), dev.alloc(4 * n + 4096)
     dev.fill(do, 7.0, n + 1024)
     dev.conv2d_bwd_weight(do, dg, dx, N, C_in, H, W, C_out, Ho, Wo, KH, KW, stride, pad)
+    _run.kernels = dev.launched(2)
     got = dev.download(do, (n + 1024,))
     assert (got[n:] == 7.0).all()  # nothing is stored past the gradient
     for b in (dx, dg, do):
@@ -83,3 +84,19 @@ def test_wgrad_split_non_finite(dev, stride):
     for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
         err = oracle.normwise_error(np.where(part, got, 0).astype(np.float64) * scale, np.where(part, ref, 0) * scale)
         assert err <= oracle.tolerance(dy[0, 0].size * 16)
+
+
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("exponent", [0, -118, -126, -140])
+def test_wgrad_split_small_operands(dev, exponent, stride):
+    """x, then dY, at the low end of fp32's range, the other large enough for
+    ordinary results: all 24 bits count there too."""
+    shape = (16, 64, 41, 41, 128, 3, 3, stride, 1)
+    case(f"wgrad split small operands 2^{exponent} stride {stride}")
+    for small in ("x", "dy"):
+        x, dy = _inputs(7300, *shape)
+        up, down = np.float32(2.0 ** (-exponent // 3)), np.float32(2.0) ** np.float32(exponent)
+        x, dy = (x * down, dy * up) if small == "x" else (x * up, dy * down)
+        got = _run(dev, x, dy, 3, 3, stride, 1)
+        assert any("wgrad_split" in k for k in _run.kernels), _run.kernels
+        assert two_norm_error(got, _ref(x, dy, 3, 3, stride, 1)) <= fp32_sum_error(dy[0, 0].size * 16), small
