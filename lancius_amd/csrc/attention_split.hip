@@ -336,7 +336,9 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
 
     // Sums that are not all finite (infinite or NaN inputs, values or scores
     // beyond the scaled range): the wave's key blocks again with the fp32
-    // instructions.
+    // instructions.  With a NaN in every sequence B8 H16 S=2048 D=64 causal
+    // takes 1423 us (440 without; with operands loaded one at a time 2542; the
+    // fp32 kernel alone 643), D=128 4998 (1765; 9497; 2285).
     float none = 0.0f, probe = l_part * 0.0f;
     asm("" : "+v"(none));
 #pragma unroll
@@ -356,13 +358,32 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
         for (int it = 0; it < nsteps; ++it) {
             const int blk = it * KS + grp, kb = blk * kKeys;
             if (!(blk < nblocks && (!p.causal || kb <= qw0 + 31 + off))) continue;
+            // (V's loads leave before the scores are formed, where there are
+            // registers for them: with D = 128 the main loop would spill)
+            constexpr bool AHEAD = NB < 4;
+            auto v_at = [&](int s, int e) {
+                const int key = kb + 8 * (s >> 2) + 4 * lk + (s & 3);
+                return __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(vbuf, (key * kv_stride + NB * lq + e) * 4, 0, 0));
+            };
+            float ahead[AHEAD ? 16 : 1][NB];
+            if constexpr (AHEAD) {
+#pragma unroll
+                for (int s = 0; s < 16; ++s)
+#pragma unroll
+                    for (int e = 0; e < NB; ++e) ahead[s][e] = v_at(s, e);
+            }
+            // lane half lk takes d = 8 t + 4 lk .. of each eight
             f32x16 s_acc = {};
-#pragma unroll 1
-            for (int t = 0; t < D / 2; ++t) {
-                const int d = 2 * t + lk;
-                const float kv = __builtin_bit_cast(
-                    float, __builtin_amdgcn_raw_buffer_load_b32(kbuf, ((kb + lq) * kv_stride + d) * 4, 0, 0));
-                s_acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv, qrow[d] * p.qscale, s_acc, 0, 0, 0);
+#pragma unroll 4
+            for (int t = 0; t < D / 8; ++t) {
+                const int d = 8 * t + 4 * lk;
+                const f32x4 kv = __builtin_bit_cast(
+                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(kbuf, ((kb + lq) * kv_stride + d) * 4, 0, 0));
+                const f32x4 qv = *(const f32x4*)(qrow + d);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    s_acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[i], qv[i] * p.qscale, s_acc, 0, 0, 0);
             }
             settle(s_acc);
             mask(s_acc, kb);
@@ -372,15 +393,11 @@ __global__ void __launch_bounds__(256 * KS, 2) attention_split(const AttnParams 
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o_acc[e][r] *= corr;
 #pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                const int key = kb + 8 * (s >> 2) + 4 * lk + (s & 3);
+            for (int s = 0; s < 16; ++s)
 #pragma unroll
-                for (int e = 0; e < NB; ++e) {
-                    const float v = __builtin_bit_cast(
-                        float, __builtin_amdgcn_raw_buffer_load_b32(vbuf, (key * kv_stride + NB * lq + e) * 4, 0, 0));
-                    o_acc[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, s_acc[s], o_acc[e], 0, 0, 0);
-                }
-            }
+                for (int e = 0; e < NB; ++e)
+                    o_acc[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(AHEAD ? ahead[AHEAD ? s : 0][e] : v_at(s, e), s_acc[s],
+                                                                    o_acc[e], 0, 0, 0);
 #pragma unroll
             for (int e = 0; e < NB; ++e) settle(o_acc[e]);
         }

@@ -166,29 +166,26 @@ __global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, 2) conv2d_spl
     const int mw = m0 + t.row0();
 
     // sums that are not all finite are recomputed in fp32 (split.hpp)
-    if (t.not_finite()) {
-#pragma unroll
-        for (int i = 0; i < T::TS; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                f32x16 s = {};
+    if (t.not_finite())
+        t.recompute(
+            0, K,
+            [&](int i, int k) {
                 const int row = mw + 32 * i + t.lr;
-#pragma unroll 1
-                for (int k0 = 0; k0 < K; k0 += 2) {
-                    const int k = k0 + t.lk, tap = k / p.C16, c = k - tap * p.C16;
-                    const int uh = tap / cl.kw, uw = tap - uh * cl.kw;
-                    const int hi = cl.mul * py[j] + cl.h0 + cl.dir * uh, wi = cl.mul * px[j] + cl.w0 + cl.dir * uw;
-                    const bool in = ok[j] & (c < p.C_in) & ((unsigned)hi < (unsigned)p.H) & ((unsigned)wi < (unsigned)p.W);
-                    const int ao = pick(row < p.C_out, (row * K + k) * 4, kOut);
-                    const int bo = pick(in, (pn[j] * p.C_in + c) * hw4 + (hi * p.W + wi) * 4, kOut);
-                    const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, ao, 0, 0));
-                    const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, bo, 0, 0));
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, s, 0, 0, 0);
-                }
-                settle(s);
-                t.acc[i][j] = s;
-            }
-    }
+                return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     rw, pick((row < p.C_out) & (k < K), (row * K + k) * 4, kOut), 0, 0));
+            },
+            [&](int j, int k) {  // (four channels of one tap: C16 is a multiple of 16)
+                const int tap = k / p.C16, c = k - tap * p.C16, uh = tap / cl.kw, uw = tap - uh * cl.kw;
+                const int hi = cl.mul * py[j] + cl.h0 + cl.dir * uh, wi = cl.mul * px[j] + cl.w0 + cl.dir * uw;
+                const bool in = ok[j] & (k < K) & ((unsigned)hi < (unsigned)p.H) & ((unsigned)wi < (unsigned)p.W);
+                const int off = (pn[j] * p.C_in + c) * hw4 + (hi * p.W + wi) * 4;
+                f32x4 v;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                         rx, pick(in & (c + q < p.C_in), off + q * hw4, kOut), 0, 0));
+                return v;
+            });
 
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, p.N * p.C_out * ohw4, kBufferRsrcWord3);
     const __amdgpu_buffer_rsrc_t rb =

@@ -55,24 +55,31 @@ __global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, 2) gemm_f32_s
 
     // sums that are not all finite are recomputed in fp32 (split.hpp)
     if (t.not_finite()) {
+        // four k of a row whose k are contiguous, or of a k-major operand's column
+        auto along = [&](__amdgpu_buffer_rsrc_t r, bool in, int row, int k) {
+            f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, pick(in, (row * K + k) * 4, kOut), 0, 0));
 #pragma unroll
-        for (int i = 0; i < T::TS; ++i)
+            for (int q = 0; q < 4; ++q) v[q] = k + q < k_end ? v[q] : 0.0f;
+            return v;
+        };
+        auto across = [&](__amdgpu_buffer_rsrc_t r, bool in, int col, int cols, int k) {
+            f32x4 v;
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int row = mw + 32 * i + row_of(t.lr), col = cb + 32 * j;
-                f32x16 s = {};
-#pragma unroll 1
-                for (int k0 = k_begin; k0 < k_end; k0 += 2) {
-                    const int k = k0 + t.lk;
-                    const int ao = pick(k < k_end && row < M, (TA ? k * M + row : row * K + k) * 4, kOut);
-                    const int bo = pick(k < k_end && col < N, (TB ? col * K + k : k * N + col) * 4, kOut);
-                    const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, ao, 0, 0));
-                    const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, bo, 0, 0));
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, s, 0, 0, 0);
-                }
-                settle(s);
-                t.acc[i][j] = s;
-            }
+            for (int q = 0; q < 4; ++q)
+                v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                     r, pick(in & (k + q < k_end), ((k + q) * cols + col) * 4, kOut), 0, 0));
+            return v;
+        };
+        t.recompute(
+            k_begin, k_end,
+            [&](int i, int k) {
+                const int row = mw + 32 * i + row_of(t.lr);
+                return TA ? across(ra, row < M, row, M, k) : along(ra, row < M, row, k);
+            },
+            [&](int j, int k) {
+                const int col = cb + 32 * j;
+                return TB ? along(rb, col < N, col, k) : across(rb, col < N, col, N, k);
+            });
     }
 
     // C through a buffer resource: rows past M fall past its end and columns

@@ -212,6 +212,47 @@ struct SplitTile {
                 for (int r = 0; r < 16; ++r) probe = fmaf(acc[i][j][r], none, probe);
         return __any(!(probe == 0.0f));
     }
+
+    // The wave's kept blocks with the fp32 instructions, over k in [k_begin,
+    // k_end): a(i, k) and b(j, k) give k .. k + 3 of this lane's row of block
+    // row i and column of block column j, 0 from k_end on.  A group of 8 k is
+    // loaded while the one before it is multiplied, and an operand serves
+    // every block of its row or column.  Bound by the fp32 matrix rate: with a
+    // NaN in each row 4096^3 takes 1777 us (585 without; block by block, two k
+    // at a time, 5518; fp32 kernels alone 1037), N32 64->128 3x3 56^2 310 (113;
+    // 904; 151), its weight gradient 315 (110; 747; 167).
+    template <class FA, class FB>
+    __device__ __forceinline__ void recompute(int k_begin, int k_end, const FA& a, const FB& b) {
+        f32x4 av[2][TS], bv[2][TN];
+#pragma unroll
+        for (int i = 0; i < TS; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+        auto load = [&](int s, int k) {
+#pragma unroll
+            for (int i = 0; i < TS; ++i) av[s][i] = a(i, k + 4 * lk);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bv[s][j] = b(j, k + 4 * lk);
+        };
+        auto multiply = [&](int s) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < TS; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s][i][q], bv[s][j][q], acc[i][j], 0, 0, 0);
+        };
+        load(0, k_begin);
+#pragma unroll 1
+        for (int k = k_begin; k < k_end; k += 16) {
+            load(1, k + 8);
+            multiply(0);
+            load(0, k + 16);
+            multiply(1);
+        }
+        settle(acc);
+    }
 };
 
 // Loaders of a matrix through a buffer resource: rows past it and k-major rows

@@ -195,29 +195,42 @@ __global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, 2) wgrad_spli
 
     // sums that are not all finite are recomputed in fp32 (split.hpp)
     if (t.not_finite()) {
+        struct Pixel {
+            int n, ho, wo;
+            bool in;
+        };
+        auto pixel = [&](int k) {  // the first of four in one octet
+            const int o = k >> 3, r = o / p.row_oct, n = r / p.Ho;
+            return Pixel{n, r - n * p.Ho, 8 * (o - r * p.row_oct) + (k & 7), o < o_end};
+        };
+        t.recompute(
+            8 * o_begin, 8 * o_end,
+            [&](int i, int k) {
+                const Pixel x = pixel(k);
+                const int co = mw + 32 * i + t.lr;
+                const int off = ((x.n * p.C_out + co) * HWo + x.ho * p.Wo + x.wo) * 4;
+                f32x4 v = __builtin_bit_cast(
+                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, pick(x.in & (co < p.C_out), off, kOut), 0, 0));
 #pragma unroll
-        for (int i = 0; i < T::TS; ++i)
+                for (int q = 0; q < 4; ++q) v[q] = x.wo + q < p.Wo ? v[q] : 0.0f;
+                return v;
+            },
+            [&](int j, int k) {
+                const Pixel x = pixel(k);
+                const int col = min(j0 + t.wn * WN + 32 * j + t.lr, p.J - 1), khw = p.KH * p.KW;
+                const int ci = col / khw, tap = col - ci * khw, th = tap / p.KW, tw = tap - th * p.KW;
+                const int hi = x.ho * p.stride + th - p.pad;
+                const bool row = x.in & ((unsigned)hi < (unsigned)p.H);
+                const int base = ((x.n * p.C_in + ci) * p.H + hi) * p.W;
+                f32x4 v;
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                f32x16 s = {};
-                const int co = mw + 32 * i + t.lr, col = min(j0 + t.wn * WN + 32 * j + t.lr, p.J - 1);
-                const int khw = p.KH * p.KW, ci = col / khw, tap = col - ci * khw, th = tap / p.KW, tw = tap - th * p.KW;
-#pragma unroll 1
-                for (int k0 = 8 * o_begin; k0 < 8 * o_end; k0 += 2) {
-                    const int k = k0 + t.lk, o = k >> 3, r = o / p.row_oct, wo = 8 * (o - r * p.row_oct) + (k & 7);
-                    const int n = r / p.Ho, ho = r - n * p.Ho;
-                    const int hi = ho * p.stride + th - p.pad, wi = wo * p.stride + tw - p.pad;
-                    const bool live = wo < p.Wo;
-                    const bool in = live & ((unsigned)hi < (unsigned)p.H) & ((unsigned)wi < (unsigned)p.W);
-                    const int ao = pick(live & (co < p.C_out), ((n * p.C_out + co) * HWo + ho * p.Wo + wo) * 4, kOut);
-                    const int bo = pick(in, (((n * p.C_in + ci) * p.H + hi) * p.W + wi) * 4, kOut);
-                    const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, ao, 0, 0));
-                    const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, bo, 0, 0));
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, s, 0, 0, 0);
+                for (int q = 0; q < 4; ++q) {
+                    const int wi = (x.wo + q) * p.stride + tw - p.pad;
+                    const bool in = row & (x.wo + q < p.Wo) & ((unsigned)wi < (unsigned)p.W);
+                    v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, pick(in, (base + wi) * 4, kOut), 0, 0));
                 }
-                settle(s);
-                t.acc[i][j] = s;
-            }
+                return v;
+            });
     }
 
     // rows past C_out fall past the end of this split's gradient

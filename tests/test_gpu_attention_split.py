@@ -113,3 +113,30 @@ def test_attention_split_range(dev, q_exp, k_exp, v_exp, D, causal):
     got = _run(dev, q, k, v, causal)
     assert "attention_split" in _run.kernel, _run.kernel
     assert two_norm_error(got, _ref(q, k, v, causal)) <= fp32_sum_error(shape[2]) + 4 * fp32_sum_error(D)
+
+
+@pytest.mark.parametrize("block", [4, 5])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+def test_attention_split_non_finite_two_groups(dev, D, causal, block):
+    """One group of waves (even or odd key blocks) recomputes in fp32 and
+    hands over to, or takes from, the group that did not."""
+    B, S, H = 1, 1100, 16
+    case(f"attention split non-finite, two groups, D={D} causal={causal} block {block}")
+    q, k, v = _inputs(5100 + D, B, S, S, H, H, D)
+    key = 32 * block + 5
+    v[0, key, 3, 4] = np.float32(3.4e38)       # finite everywhere, beyond the scaled range
+    v[0, key, 5, 6] = np.inf
+    k[0, key, 7, 8] = np.float32(2.0 ** 113)   # scores of +-2^113 or so: the key takes all or nothing
+    got, ref = _run(dev, q, k, v, causal), _ref(q, k, v, causal)
+    assert _run.kernel == f"attention_split D={D} x2"
+    if causal:  # (probability 0 times infinity is NaN where the kernel reaches a masked key)
+        got[0, :key, 5, 6] = ref[0, :key, 5, 6] = 0.0
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert inf.any() and np.array_equal(got[inf], ref[inf].astype(np.float32))
+    big = np.isfinite(ref) & (np.abs(ref) > 1e20)
+    assert big.any()
+    for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
+        err = two_norm_error(got[part].astype(np.float64) * scale, ref[part] * scale)
+        assert err <= fp32_sum_error(S) + 4 * fp32_sum_error(D)

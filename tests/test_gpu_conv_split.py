@@ -151,3 +151,43 @@ def test_conv_split_small_operands(dev, what, exponent):
             ref = F.conv_transpose2d(x64, w64, None, stride, 1, output_padding=stride - 1)
         assert "conv2d_split" in kernel, kernel
         assert two_norm_error(got, ref.numpy()) <= fp32_sum_error(9 * (C_in if what == "forward" else C_out)), small
+
+
+# as FORWARD and GRADIENT, with the kernel
+RECOMPUTED = [
+    ("forward", 40, 32, 31, 33, 132, 3, 3, 1, 1, "conv2d_split 128x128 x1"),
+    ("forward", 32, 64, 56, 56, 128, 3, 3, 2, 1, "conv2d_split 128x128 x2"),
+    ("forward", 8, 90, 40, 40, 200, 3, 3, 1, 1, "conv2d_split 128x128 x2"),   # channels padded to 96
+    ("forward", 10, 64, 56, 56, 64, 3, 3, 1, 1, "conv2d_split 64x128 x2"),
+    ("gradient", 8, 128, 40, 36, 128, 3, 3, 1, 1, "conv2d_split 128x128 x2"),
+    ("gradient", 24, 128, 57, 55, 72, 3, 3, 2, 1, "conv2d_split 128x128 x1"),
+    ("gradient", 8, 64, 57, 55, 100, 3, 3, 2, 1, "conv2d_split 64x128 x2"),
+]
+
+
+@pytest.mark.parametrize("what,N,C_in,H,W,C_out,KH,KW,stride,pad,kernel", RECOMPUTED)
+def test_conv_split_recomputes_non_finite(dev, what, N, C_in, H, W, C_out, KH, KW, stride, pad, kernel):
+    """The tiles that hold infinities, NaN and values beyond the scaled range
+    are computed again in fp32, in each form of the kernel."""
+    case(f"conv split recompute {what} {N} {C_in}->{C_out} {H}x{W} stride {stride}")
+    w = prng.normal(6401, (C_out, C_in, KH, KW), std=0.06)
+    x = prng.normal(6400, (N, C_in, H, W) if what == "forward" else (N, C_out, _out(H, KH, stride, pad), _out(W, KW, stride, pad)))
+    x[0, 3, 5, 7], x[2, -1, -1, -1], x[-1, 0, 0, 0] = np.inf, np.nan, -np.inf
+    x[4, 10, 11, 12] = np.float32(3.4e38)
+    (w[7, 10] if what == "forward" else w[10, 7])[...] *= np.float32(2.0 ** -20)
+    x64, w64 = torch.from_numpy(x).double(), torch.from_numpy(w).double()
+    if what == "forward":
+        got, ran = _forward(dev, x, w, None, stride, pad, ACT_NONE, C_in % 16 == 0 and C_out % 4 == 0), _forward.kernel
+        ref = F.conv2d(x64, w64, None, stride, pad).numpy()
+    else:
+        got, ran = _bwd_input(dev, x, w, H, W, stride, pad), _bwd_input.kernel
+        over = ((H + 2 * pad - KH) % stride, (W + 2 * pad - KW) % stride)
+        ref = F.conv_transpose2d(x64, w64, None, stride, pad, output_padding=over).numpy()
+    assert ran == kernel
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert inf.any() and np.array_equal(got[inf], ref[inf].astype(np.float32))
+    big = np.isfinite(ref) & (np.abs(ref) > 1e20)
+    assert big.any()
+    for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
+        assert two_norm_error(got[part].astype(np.float64) * scale, ref[part] * scale) <= fp32_sum_error(w[0].size)

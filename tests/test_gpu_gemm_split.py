@@ -105,7 +105,7 @@ def test_gemm_split_small_operands(dev, M, K, N, exponent, layout):
 
 
 @pytest.mark.parametrize("layout", ["NN", "TN", "NT"])
-@pytest.mark.parametrize("M,K,N", [(1031, 289, 4093), (3456, 64, 3712), (512, 4096, 512)])
+@pytest.mark.parametrize("M,K,N", [(1031, 289, 4093), (3456, 64, 3712), (512, 4096, 512), (1153, 289, 2303)])
 def test_gemm_split_non_finite(dev, M, K, N, layout):
     """Infinities, NaN and values above the largest bf16 give what fp32
     arithmetic gives: an infinite input spoils its own row or column only,

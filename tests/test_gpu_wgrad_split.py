@@ -100,3 +100,25 @@ def test_wgrad_split_small_operands(dev, exponent, stride):
         got = _run(dev, x, dy, 3, 3, stride, 1)
         assert any("wgrad_split" in k for k in _run.kernels), _run.kernels
         assert two_norm_error(got, _ref(x, dy, 3, 3, stride, 1)) <= fp32_sum_error(dy[0, 0].size * 16), small
+
+
+@pytest.mark.parametrize("shape,kernel", [((16, 64, 41, 41, 128, 3, 3, 2, 1), "wgrad_split 128x128"),
+                                          ((16, 64, 41, 40, 128, 3, 3, 1, 1), "wgrad_split 128x128"),
+                                          ((12, 40, 45, 33, 60, 5, 5, 2, 2), "wgrad_split 64x128")])
+def test_wgrad_split_recomputes_non_finite(dev, shape, kernel):
+    """The tiles that an infinite, NaN or out-of-range value reaches are
+    computed again in fp32: rows that are no whole octets, strides, both tiles."""
+    case(f"wgrad split recompute {shape}")
+    x, dy = _inputs(7400, *shape)
+    x[0, 3, 0, 0], x[5, 20, 17, 18] = np.inf, np.nan
+    dy[7, 9, -1, -1] = -np.inf
+    x[3, 30, 11, 12] = np.float32(3.4e38)
+    got, ref = _run(dev, x, dy, *shape[5:]), _ref(x, dy, *shape[5:])
+    assert kernel in _run.kernels
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert inf.any() and np.array_equal(got[inf], ref[inf].astype(np.float32))
+    big = np.isfinite(ref) & (np.abs(ref) > 1e20)
+    assert big.any()
+    for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
+        assert two_norm_error(got[part].astype(np.float64) * scale, ref[part] * scale) <= fp32_sum_error(dy[0, 0].size * shape[0])
