@@ -1220,7 +1220,8 @@ struct GemmPlan {
     double us;
 };
 
-GemmPlan gemm_plan(size_t count, size_t M, size_t K, size_t N, bool plain, bool vec) {
+// may_split: the split-product kernels take the product (without, the fp32 kernels' cost).
+GemmPlan gemm_plan(size_t count, size_t M, size_t K, size_t N, bool plain, bool vec, bool may_split) {
     const double k = (double)K;
     auto tiles = [&](size_t bm, size_t bn) { return count * ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     auto rounds = [](size_t t) { return (double)((t + 255) / 256); };
@@ -1238,6 +1239,7 @@ GemmPlan gemm_plan(size_t count, size_t M, size_t K, size_t N, bool plain, bool 
     const double out_bytes = 4.0 * (double)count * M * N;
     fp32 += out_bytes / 6e6;
     GemmPlan best{-1, 1, fp32};
+    if (!may_split) return best;
     if (t128 >= 768) best.us = 1e30;  // split products are ahead there down to K = 16 (4096 x 48 x 4096: 27 -> 18)
     auto offer = [&](int tile, size_t splits, size_t t, double start, double per_k, double after) {
         const double full = (double)(t / 256), fill = (double)(t % 256) / 256;
@@ -1363,27 +1365,26 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
         }
     }
 
-    const GemmPlan plan = gemm_plan(count, M, K, N, !ta && !tb, vec);
-    if (small_plan.us < plan.us) return run_small();
     // Products large enough for the bf16 matrix cores' split products
     // (gemm_split.hip); both operands transposed, or one beyond 32-bit
     // offsets, stay with the fp32 kernels.
-    if (!(ta && tb) && split_fits && (K >= 32 || big_tiles >= 768)) {
-        if (plan.tile >= 0 &&
-            (plan.splits == 1 || fixed || workspace_ready(ctx, count * plan.splits * M * N * sizeof(float)))) {
-            const size_t steps = (K + 31) / 32, chunk = (steps + plan.splits - 1) / plan.splits;
-            p.splits = (int)((steps + chunk - 1) / chunk);  // no empty K range
-            p.kchunk = (int)(chunk * 32);
-            if (p.splits > 1) {
-                void* ws = nullptr;
-                if (int rc = partials(ctx, fixed, count * p.splits * M * N * sizeof(float), &ws)) return rc;
-                p.ws = (float*)ws;
-            }
-            if (int rc = launch_gemm_split(ctx, p, (int)count, ta, tb, plan.tile)) return rc;
-            if (p.splits > 1)
-                if (int rc = launch_splitk_reduce(ctx, p, (int)count)) return rc;
-            return ok();
+    const bool may_split = !(ta && tb) && split_fits && (K >= 32 || big_tiles >= 768);
+    const GemmPlan plan = gemm_plan(count, M, K, N, !ta && !tb, vec, may_split);
+    if (small_plan.us < plan.us) return run_small();
+    if (plan.tile >= 0 &&
+        (plan.splits == 1 || fixed || workspace_ready(ctx, count * plan.splits * M * N * sizeof(float)))) {
+        const size_t steps = (K + 31) / 32, chunk = (steps + plan.splits - 1) / plan.splits;
+        p.splits = (int)((steps + chunk - 1) / chunk);  // no empty K range
+        p.kchunk = (int)(chunk * 32);
+        if (p.splits > 1) {
+            void* ws = nullptr;
+            if (int rc = partials(ctx, fixed, count * p.splits * M * N * sizeof(float), &ws)) return rc;
+            p.ws = (float*)ws;
         }
+        if (int rc = launch_gemm_split(ctx, p, (int)count, ta, tb, plan.tile)) return rc;
+        if (p.splits > 1)
+            if (int rc = launch_splitk_reduce(ctx, p, (int)count)) return rc;
+        return ok();
     }
 
     // Configurations (BM x BN / BK, k-groups): 2 = 64x64/16, 6 = 128x128/16

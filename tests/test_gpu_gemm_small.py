@@ -21,6 +21,7 @@ def _run(dev, A, B, M, K, N, ta, tb, bias=None, act=ACT_NONE, residual=None, shi
     db = dev.upload(bias) if bias is not None else None
     dR = dev.upload(residual) if residual is not None else None
     dev.gemm_ex(dC, dA.ptr + 4 * shift, dB.ptr + 4 * shift, M, K, N, trans_a=ta, trans_b=tb, bias=db, act=act, residual=dR)
+    _run.kernel = dev.launched()[0]
     got = dev.download(dC, (M * N + 1024,))
     assert (got[M * N:] == 7.0).all()  # nothing is stored past C
     for b in (dA, dB, dC, db, dR):
@@ -51,6 +52,19 @@ def test_gemm_small_shapes(dev, M, K, N, layout):
     if R is not None:
         ref = ref + R
     assert oracle.normwise_error(got, ref) <= oracle.tolerance(K)
+
+
+@pytest.mark.parametrize("layout,small", [("TT", True), ("NT", False)])
+def test_gemm_small_against_what_the_layout_can_take(dev, layout, small):
+    """8080 x 2222 x 17: split products are ahead of small tiles, which are
+    ahead of the fp32 kernels; with both operands transposed only the last two
+    are there."""
+    M, K, N = 8080, 2222, 17
+    case(f"gemm small or split {layout}")
+    A, B = prng.normal(2250, (M, K)), prng.normal(2251, (K, N))
+    got = _run(dev, A, B, M, K, N, layout[0] == "T", True)
+    assert ("gemm_f32_small" in _run.kernel) == small, _run.kernel
+    assert oracle.normwise_error(got, A.astype(np.float64) @ B.astype(np.float64)) <= oracle.tolerance(K)
 
 
 @pytest.mark.parametrize("shift", [1, 2, 3])
