@@ -24,6 +24,7 @@
 #include <cmath>
 
 #include "conv.hpp"
+#include "split.hpp"
 
 namespace lancius {
 namespace {
@@ -1229,7 +1230,7 @@ bool use_split(lancius_hip_ctx* ctx, const ConvParams& q, ConvSplitParams* sp) {
         sp->small_tile = tile;
         return true;
     }
-    return split < fp32;
+    return split < fp32 && (size_t)q.Kdim >= kSplitLeast;
 }
 
 // One launch per run of images whose input stays under 2 GiB (the direct
@@ -1399,7 +1400,7 @@ extern "C" int lancius_hip_conv2d_bwd_input_f32(lancius_hip_ctx* ctx, float* dx,
         if (C_out * K_h * K_w > 12 && stride <= 16 && K_h < (1u << 15) && K_w < (1u << 15) && C_out > 0 && pad < (1u << 30) && conv_split_fits(sp) &&
             workspace_ready(ctx, conv_split_weight_bytes(sp))) {
             int tile;
-            if (conv_small_plan(sp, &tile) < conv_split_us(sp)) sp.small_tile = tile;
+            if (conv_small_plan(sp, &tile) < conv_split_us(sp) || C_out < kSplitLeast) sp.small_tile = tile;
             const int rc = launch_conv_split(ctx, sp, w);
             return rc ? rc : ok();
         }
@@ -1449,7 +1450,7 @@ extern "C" int lancius_hip_conv2d_bwd_weight_f32(lancius_hip_ctx* ctx, float* dw
     WgradSplitParams sp{dw, dy, x, (int)N, (int)C_in, (int)H, (int)W, (int)C_out, (int)H_out, (int)W_out, (int)K_h, (int)K_w,
                         (int)stride, (int)pad, (int)J, 0, 0, 0, 0, 0, 0};
     if (N > 0 && H_out > 0 && W_out > 0 && H > 0 && W > 0 && N * C_in < ((size_t)1 << 30) && N * C_out < ((size_t)1 << 30) &&
-        stride < (1u << 15) && pad < (1u << 15) && wgrad_split_fits(sp)) {
+        stride < (1u << 15) && pad < (1u << 15) && N * H_out * W_out >= kSplitLeast && wgrad_split_fits(sp)) {
         double us = 0.0;
         wgrad_split_plan(sp, (size_t)cu_count(ctx), &us);
         if (workspace_ready(ctx, sp.splits > 1 ? (size_t)sp.splits * C_out * J * sizeof(float) : 0) &&

@@ -25,6 +25,7 @@
 #include <mutex>
 
 #include "gemm.hpp"
+#include "split.hpp"
 
 namespace lancius {
 namespace {
@@ -1045,8 +1046,8 @@ launched:
 // Transposed operands are built for the two default tile shapes only.
 // Configurations 6 and 8 run grids of at least 256 tiles, which never split
 // K; with plain operands, configuration 6 (at least 768 tiles) is left with
-// operands beyond the split-product kernels' 32-bit offsets, and is built
-// with scalar loads only.
+// operands beyond the split-product kernels' 32-bit offsets and K < 3, and is
+// built with scalar loads only.
 template <bool TA, bool TB>
 int launch_by_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec, int cfg) {
     if constexpr (TA || TB) {
@@ -1367,8 +1368,9 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
 
     // Products large enough for the bf16 matrix cores' split products
     // (gemm_split.hip); both operands transposed, or one beyond 32-bit
-    // offsets, stay with the fp32 kernels.
-    const bool may_split = !(ta && tb) && split_fits && (K >= 32 || big_tiles >= 768);
+    // offsets, stay with the fp32 kernels, and so do sums of one or two
+    // products, for their rounding (split.hpp).
+    const bool may_split = !(ta && tb) && split_fits && (K >= 32 || (big_tiles >= 768 && K >= kSplitLeast));
     const GemmPlan plan = gemm_plan(count, M, K, N, !ta && !tb, vec, may_split);
     if (small_plan.us < plan.us) return run_small();
     if (plan.tile >= 0 &&
@@ -1391,7 +1393,7 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
     // built for 4 workgroups per CU, 7 = 128x128/32 x2, 8 = 128x128/32 x4,
     // 9 = 64x64/64 x4.  Chosen by the number of 128x128 tiles (one per CU
     // fills the chip once), measured on MI355X:
-    //  * >= 768: 6 (operands beyond 32-bit offsets);
+    //  * >= 768: 6 (operands beyond 32-bit offsets, K < 3);
     //  * 384 .. 767: 7 (two 8-wave workgroups per CU);
     //  * 256 .. 383: 8, 16 waves on the CU's one tile (4096x1024x1024: 110 ->
     //    103 us);
@@ -1458,7 +1460,7 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
         p.ws = (float*)ws;
     }
     // plain configuration-6 grids come here only with operands beyond 32-bit
-    // offsets: scalar loads
+    // offsets or K < 3: scalar loads
     if (cfg == 6 && plain) vec = false;
     int rc;
     if (ta && tb)

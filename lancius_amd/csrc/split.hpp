@@ -5,8 +5,13 @@
 // differences are exact in fp32, and 3 x 8 significand bits cover its 24).
 // A product x y is then formed from six bf16 products,
 //     hh' + (hm' + mh') + (mm' + hl' + lh'),
-// each exact in the fp32 accumulator's input.  The three products left out
-// (ml', lm', ll') are below 2^-26 of x y, under half an fp32 ulp.  The
+// each exact in the fp32 accumulator's input.  Of the three products left out
+// ml' and lm' reach 2^-25 of x y each (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|): 2^-24
+// at most, half an fp32 ulp or one, and 2^-27.4 rms.  A single product is
+// then not always the correctly rounded one, so sums of one or two stay with
+// the fp32 kernels (kSplitLeast); from three on the fp32 chain's own roundings
+// are the larger error (3584 x K x 3584, two-norm, fp32 and split: K = 1 2.53e-8,
+// 3.45e-8; 2 3.12e-8, 3.38e-8; 3 3.57e-8, 3.29e-8; 16 7.4e-8, 3.4e-8).  The
 // accumulator is fp32 as before, and the six are summed from the smallest
 // terms up.  v_mfma_f32_32x32x16_bf16 does 16 times the multiply-adds per
 // cycle of v_mfma_f32_32x32x2_f32, so six of them leave a factor of 2.7 in
@@ -45,6 +50,8 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
 }
 
+// Products that a sum has at least.
+constexpr size_t kSplitLeast = 3;
 constexpr float kSplitUp = 0x1p16f, kSplitDown = 0x1p-32f;
 
 // The three parts of x; split8_up: of x as scaled.

@@ -9,6 +9,7 @@ import torch.nn.functional as F
 import oracle
 from lancius_amd import ACT_NONE, ACT_RELU, prng
 from tests.conftest import case, fp32_sum_error, two_norm_error
+from tests.test_gpu_gemm_split import ROUNDING
 
 pytestmark = pytest.mark.gpu
 
@@ -191,3 +192,17 @@ def test_conv_split_recomputes_non_finite(dev, what, N, C_in, H, W, C_out, KH, K
     assert big.any()
     for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
         assert two_norm_error(got[part].astype(np.float64) * scale, ref[part] * scale) <= fp32_sum_error(w[0].size)
+
+
+def test_conv_gradient_of_few_channels_rounds_as_fp32(dev):
+    """dy of two channels at stride 2: a quarter of the elements see one tap,
+    two products, and the call stays with the fp32 instructions."""
+    N, C_in, C_out, H, W, stride, pad = 24, 130, 2, 64, 64, 2, 1
+    case("conv gradient of two channels")
+    dy = prng.normal(6700, (N, C_out, _out(H, 3, stride, pad), _out(W, 3, stride, pad)))
+    w = prng.normal(6701, (C_out, C_in, 3, 3))
+    got = _bwd_input(dev, dy, w, H, W, stride, pad)
+    assert "conv2d_small" in _bwd_input.kernel
+    centre = np.einsum("nchw,ci->nihw", dy.astype(np.float64), w[:, :, 1, 1].astype(np.float64))
+    # both products and their sum round; a tenth for the few random weights
+    assert two_norm_error(got[:, :, ::2, ::2], centre) <= 1.1 * ROUNDING * np.sqrt((1 + 1 + 2) / 2)

@@ -67,6 +67,28 @@ def test_gemm_split_shapes(dev, M, K, N, what, layout):
     assert np.abs(got - ref).max() <= 60 * oracle.tolerance(K) * scale
 
 
+# What rounding to fp32 does to random values, two-norm (0.42 ulp / 2).  An fp32 chain of K
+# products rounds the first product and each sum after it, which grow as sqrt(i):
+# ROUNDING * sqrt((1 + 2 + ... + K) / K).
+ROUNDING = 0.43 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("layout", ["NN", "TN", "NT"])
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 16, 33])
+def test_gemm_few_products_round_as_fp32(dev, K, layout):
+    """Six bf16 products leave out up to 2^-24 of each product: one or two of
+    them round better with the fp32 instructions and stay there."""
+    M, N = 3585, 3590
+    case(f"gemm of {K} products {layout}")
+    A, B = prng.normal(71, (M, K)), prng.normal(72, (K, N))
+    ta, tb = layout[0] == "T", layout[1] == "T"
+    got = _run(dev, np.ascontiguousarray(A.T) if ta else A, np.ascontiguousarray(B.T) if tb else B, M, K, N, ta, tb)
+    assert ("gemm_f32_split" in _run.kernels[0]) == (K >= 3)
+    assert two_norm_error(got, A.astype(np.float64) @ B.astype(np.float64)) <= ROUNDING * np.sqrt((K + 1) / 2)
+    if K == 1:
+        assert np.array_equal(got, A * B)
+
+
 def test_gemm_split_k_is_repeatable(dev):
     M, K, N = 512, 4096, 512
     A, B = prng.normal(1, (M, K)), prng.normal(2, (K, N))

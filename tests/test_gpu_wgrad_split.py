@@ -9,6 +9,7 @@ import torch.nn.functional as F
 import oracle
 from lancius_amd import prng
 from tests.conftest import case, fp32_sum_error, two_norm_error
+from tests.test_gpu_gemm_split import ROUNDING
 
 pytestmark = pytest.mark.gpu
 
@@ -122,3 +123,22 @@ def test_wgrad_split_recomputes_non_finite(dev, shape, kernel):
     assert big.any()
     for part, scale in ((big, 2.0 ** -100), (np.isfinite(ref) & ~big, 1.0)):
         assert two_norm_error(got[part].astype(np.float64) * scale, ref[part] * scale) <= fp32_sum_error(dy[0, 0].size * shape[0])
+
+
+@pytest.mark.parametrize("images", [1, 2, 3])
+def test_wgrad_few_products_round_as_fp32(dev, images):
+    """A gradient over one or two pixels is one or two products an element and
+    stays with the fp32 kernels."""
+    x, dy = prng.normal(7500, (images, 96, 1, 1)), prng.normal(7501, (images, 160, 1, 1))
+    case(f"wgrad over {images} pixels")
+    got = _run(dev, x, dy, 1, 1, 1, 0)[:, :, 0, 0]
+    assert ("wgrad_split" in _run.kernels[0]) == (images >= 3)
+    x, dy = x[:, :, 0, 0], dy[:, :, 0, 0]
+    terms = [np.outer(dy[n].astype(np.float64), x[n].astype(np.float64)) for n in range(images)]
+    ref = sum(terms)
+    if images == 1:
+        assert np.array_equal(got, dy.T * x)
+    elif images == 2:  # both products and their sum round; a tenth for the few random numbers
+        room = np.sqrt(sum(np.sum(t ** 2) for t in terms + [ref]) / np.sum(ref ** 2))
+        assert two_norm_error(got, ref) <= 1.1 * ROUNDING * room
+    assert two_norm_error(got, ref) <= fp32_sum_error(images)
