@@ -993,18 +993,18 @@ int launch_splitk_reduce(lancius_hip_ctx* ctx, const GemmParams& p, int count) {
 }
 
 // SPLITS: the configuration can be chosen for a split K (grids under 256
-// tiles); VECS: with float4 operand loads (false where the dispatch sends
+// tiles); WHOLE: for a whole one; VECS: with float4 operand loads (false where the dispatch sends
 // every float4-shaped case of the configuration to a direct kernel).  Only
 // the variants the dispatch can reach are built.
 template <int BM, int BN, int BK, int WGM, int WGN, int OCC = 1, bool TA = false, bool TB = false, int KG = 1,
-          bool SPLITS = true, bool VECS = true>
+          bool SPLITS = true, bool VECS = true, bool WHOLE = true>
 int launch_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec) {
     constexpr int SOCC = KG > 1 ? OCC : 1;  // occupancy hint of the split and scalar variants
     p.tiles_m = (uint32_t)((p.M + BM - 1) / BM);
     p.tiles_n = (uint32_t)((p.N + BN - 1) / BN);
     dim3 grid(p.tiles_m * p.tiles_n, (unsigned)p.splits, (unsigned)count);
     const bool split = p.splits > 1;
-    LANCIUS_REQUIRE((SPLITS || !split) && (VECS || !vec), LANCIUS_HIP_ERR_INTERNAL,
+    LANCIUS_REQUIRE((SPLITS || !split) && (WHOLE || split) && (VECS || !vec), LANCIUS_HIP_ERR_INTERNAL,
                     "gemm: configuration %dx%d/%d without this variant (split %d, vec %d)", BM, BN, BK, (int)split,
                     (int)vec);
     const dim3 block(kThreads * KG);
@@ -1018,7 +1018,7 @@ int launch_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec) {
             goto launched;
         }
     }
-    if constexpr (VECS) {
+    if constexpr (VECS && WHOLE) {
         if (vec) {
             name = NAME("float4");
             hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, BK, WGM, WGN, true, false, OCC, TA, TB, KG>), grid, block, 0,
@@ -1034,9 +1034,11 @@ int launch_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec) {
             goto launched;
         }
     }
-    name = NAME("scalar");
-    hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, BK, WGM, WGN, false, false, SOCC, TA, TB, KG>), grid, block, 0,
-                       ctx->stream, p);
+    if constexpr (WHOLE) {
+        name = NAME("scalar");
+        hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, BK, WGM, WGN, false, false, SOCC, TA, TB, KG>), grid, block, 0,
+                           ctx->stream, p);
+    }
 launched:
 #undef NAME
     if (int rc = check_launch(name)) return rc;
@@ -1055,7 +1057,8 @@ int launch_by_cfg(lancius_hip_ctx* ctx, GemmParams& p, int count, bool vec, int 
         return launch_cfg<128, 128, 16, 2, 2, 4, TA, TB, 1, false>(ctx, p, count, vec);
     } else {
         switch (cfg) {
-            case 2: return launch_cfg<64, 64, 16, 2, 2>(ctx, p, count, vec);
+            // (without a K to split such grids are gemm_small.hip's)
+            case 2: return launch_cfg<64, 64, 16, 2, 2, 1, false, false, 1, true, true, false>(ctx, p, count, vec);
             case 7: return launch_cfg<128, 128, 32, 2, 2, 2, false, false, 2>(ctx, p, count, vec);
             case 8: return launch_cfg<128, 128, 32, 2, 2, 1, false, false, 4, false>(ctx, p, count, vec);
             case 9: return launch_cfg<64, 64, 64, 2, 2, 1, false, false, 4>(ctx, p, count, vec);
