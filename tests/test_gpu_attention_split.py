@@ -3,6 +3,7 @@ ragged query and key counts at the edges of its tiles, each head dim, both
 grids (one tile per CU, and more), and non-finite inputs, against fp64."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from lancius_amd import prng
@@ -64,6 +65,86 @@ def test_attention_split_shapes(dev, shape, D, causal):
     q, k, v = _inputs(4000 + D, *shape, D)
     got = _run(dev, q, k, v, causal)
     assert oracle.normwise_error(got, _ref(q, k, v, causal)) <= oracle.tolerance(max(shape[2], D))
+
+
+# grids of at most 256 tiles whatever D (D = 64: more than 256 of 64 queries):
+# two groups of waves take the even and the odd key blocks
+TWO_GROUPS = [
+    (1, 1100, 1100, 16, 16),  # an even number of key blocks less four keys
+    (1, 1089, 1121, 16, 4),   # an odd number and one key, a last tile of 65 queries
+    (2, 640, 1000, 16, 8),
+]
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("shape", TWO_GROUPS, ids=["x".join(map(str, s)) for s in TWO_GROUPS])
+def test_attention_split_two_groups(dev, shape, D, causal):
+    case(f"attention split, two groups, {shape} D={D} causal={causal}")
+    q, k, v = _inputs(4200 + D, *shape, D)
+    got = _run(dev, q, k, v, causal)
+    assert _run.kernel == f"attention_split D={D} x2"
+    assert two_norm_error(got, _ref(q, k, v, causal)) <= fp32_sum_error(shape[2]) + 4 * fp32_sum_error(D)
+
+
+def _low(rng_seed, n):
+    """n numbers and their first two bf16 parts."""
+    x = torch.from_numpy(prng.normal(rng_seed, (n,)))
+    h = x.bfloat16().float()
+    return tuple(t.numpy() for t in (x, h, (x - h).bfloat16().float()))
+
+
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+def test_attention_split_scores_keep_their_low_products(dev, D):
+    """Scores whose four terms x y - h yh - h ym - m yh (h, m: the first two
+    bf16 parts) leave what the parts' last products add, about 2^-16, scaled
+    up to ordinary size: without one of hl', mm', lh' a score is off by as much
+    as it is; with them by the fp32 sum's rounding, 2^-24 of xy, 2^-8 of it."""
+    B, S, H = 9, 150, 16
+    case(f"attention split low products of the scores D={D}")
+    n = B * S * H
+    x, xh, xm = _low(4301, n * D // 4)
+    y, yh, ym = _low(4302, n * D // 4)
+    q = np.stack([x, -xh, -xh, -xm], -1).reshape(B, S, H, D)
+    k = np.stack([y, yh, ym, yh], -1).reshape(B, S, H, D)
+    # one key row per head serves every query: the terms have to belong together
+    k[:] = k[:, :1]
+    q64 = q.reshape(B, S, H, D // 4, 4).astype(np.float64)
+    y64 = k.reshape(B, S, H, D // 4, 4)[:, :1].astype(np.float64)
+    assert np.abs((q64 * y64).sum(-1)).max() < 2.0 ** -11
+    # half of the keys are zero: their score is 0, the others' what is left
+    k[:, ::2] = 0.0
+    v = prng.normal(4303, (B, S, H, D))
+    scale = 2.0 ** 16 / np.sqrt(D)
+    dq, dk, dv, do = dev.upload(q), dev.upload(k), dev.upload(v), dev.alloc(q.nbytes)
+    dev.attention_gqa(do, dq, dk, dv, B, S, S, H, H, D, False, scale)
+    assert "attention_split" in dev.launched()[0]
+    got = dev.download(do, q.shape)
+    for b in (dq, dk, dv, do):
+        b.free()
+    ref = _ref(q * np.float64(scale * np.sqrt(D)), k, v, False)
+    assert two_norm_error(got, ref) <= 2.0 ** -6
+
+
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+def test_attention_split_keeps_constant_values(dev, D):
+    """The weighted mean of one value is that value: probabilities lose no more
+    than their own rounding on the way into the products, and V nothing (a row
+    that sees one key is V bit for bit)."""
+    B, S, H = 9, 150, 16
+    case(f"attention split constant values D={D}")
+    q, k, v = _inputs(4400 + D, B, S, S, H, H, D)
+    v[:] = v[:, :1]
+    got = _run(dev, q, k, v, True)
+    assert "attention_split" in _run.kernel
+    assert np.array_equal(got[:, 0], v[:, 0])
+    # Rows of up to eight keys: numerator, sum, reciprocal and product round by
+    # at most 2^-24 each, the numerator's matrix sum up to three times (1.0 rms
+    # and 4.1 at most measured, in 2^-24); a probability short of its third part
+    # is off by 2^-18 or so, 38 rms of one key.  Later rows round once more a step.
+    err = 2.0 ** 24 * np.abs(got.astype(np.float64) - v) / np.abs(v)
+    assert err[:, 1:8].max() <= 6 and np.sqrt(np.mean(err[:, 1:8] ** 2)) <= 2
+    assert err.max() <= 6 + 2 * S / 32
 
 
 @pytest.mark.parametrize("causal", [False, True])

@@ -58,52 +58,74 @@ def _bwd_input(dev, dy, w, H, W, stride, pad):
     return got[:n].reshape(N, C_in, H, W)
 
 
-# (N, C_in, H, W, C_out, KH, KW, stride, pad, packed)
+# (N, C_in, H, W, C_out, KH, KW, stride, pad, packed, kernel: channels x pixels of a tile x groups of waves)
 FORWARD = [
-    (9, 64, 40, 36, 128, 3, 3, 1, 1, True),     # whole tiles, a tile a CU or less
-    (40, 32, 31, 33, 132, 3, 3, 1, 1, True),    # four channels past a tile, two tiles a CU
-    (3, 48, 57, 55, 96, 5, 5, 2, 2, True),      # stride 2, ragged pixels
-    (2, 37, 40, 41, 70, 3, 5, 1, 2, False),     # channels padded to 48, an oblong filter
-    (2, 96, 30, 30, 24, 7, 7, 3, 0, False),     # few output channels, stride 3, no padding
-    (1, 13, 64, 64, 51, 5, 5, 1, 2, False),
+    (9, 64, 40, 36, 128, 3, 3, 1, 1, True, "conv2d_split 128x128 x2"),     # whole tiles, a tile a CU or less
+    (40, 32, 31, 33, 132, 3, 3, 1, 1, True, "conv2d_split 128x128 x1"),    # four channels past a tile, two tiles a CU
+    (24, 48, 57, 55, 96, 5, 5, 2, 2, True, "conv2d_split 128x128 x2"),     # stride 2, ragged pixels
+    (64, 96, 60, 61, 128, 3, 3, 3, 0, True, "conv2d_split 128x128 x2"),    # stride 3, no padding
+    (32, 37, 40, 41, 70, 3, 5, 1, 2, False, "conv2d_split 128x128 x1"),    # channels padded to 48, an oblong filter
+    (8, 90, 40, 40, 200, 3, 3, 1, 1, False, "conv2d_split 128x128 x2"),    # channels padded to 96
+    (10, 64, 56, 56, 64, 3, 3, 1, 1, True, "conv2d_split 64x128 x2"),      # 64-channel tiles
+    (20, 64, 56, 56, 60, 3, 3, 1, 1, True, "conv2d_split 64x128 x1"),      # four channels short of one
+    (10, 13, 64, 64, 51, 5, 5, 1, 2, False, "conv2d_split 64x128 x1"),     # both channel counts ragged
+    (3, 48, 57, 55, 96, 5, 5, 2, 2, True, "conv2d_small 32x32"),           # few pixels of the same
+    (2, 37, 40, 41, 70, 3, 5, 1, 2, False, "conv2d_small 32x32"),
+    (2, 96, 30, 30, 24, 7, 7, 3, 0, False, "conv2d_small 16x16"),
+    (1, 13, 64, 64, 51, 5, 5, 1, 2, False, "conv2d_small 32x32"),
 ]
 
 
-@pytest.mark.parametrize("N,C_in,H,W,C_out,KH,KW,stride,pad,packed", FORWARD)
-def test_conv_split_forward(dev, N, C_in, H, W, C_out, KH, KW, stride, pad, packed):
+@pytest.mark.parametrize("N,C_in,H,W,C_out,KH,KW,stride,pad,packed,kernel", FORWARD)
+def test_conv_split_forward(dev, N, C_in, H, W, C_out, KH, KW, stride, pad, packed, kernel):
     case(f"conv split forward {N} {C_in}->{C_out} {H}x{W} {KH}x{KW} stride {stride}")
     x = prng.normal(6000, (N, C_in, H, W))
     w = prng.normal(6001, (C_out, C_in, KH, KW), std=float(np.sqrt(2.0 / (C_in * KH * KW))))
     b = prng.normal(6002, (C_out,))
     act = ACT_RELU if stride == 1 else ACT_NONE
     got = _forward(dev, x, w, b, stride, pad, act, packed)
+    assert _forward.kernel == kernel
     ref = F.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), torch.from_numpy(b).double(), stride, pad)
     ref = (F.relu(ref) if act == ACT_RELU else ref).numpy()
     assert oracle.normwise_error(got, ref) <= oracle.tolerance(C_in * KH * KW)
+    if act == ACT_NONE:  # (a ReLU of a sum near 0 keeps its error and not its size)
+        assert two_norm_error(got, ref) <= fp32_sum_error(C_in * KH * KW)
 
 
-# (N, C_in, H, W, C_out, KH, KW, stride, pad)
+# (N, C_in, H, W, C_out, KH, KW, stride, pad, kernel)
 GRADIENT = [
-    (8, 64, 40, 36, 128, 3, 3, 1, 1),
-    (2, 96, 33, 31, 48, 5, 5, 1, 2),
-    (3, 40, 33, 30, 72, 3, 3, 2, 1),     # classes of different sizes
-    (2, 130, 20, 23, 37, 5, 5, 2, 2),    # dy's channels padded to 48
-    (2, 24, 32, 32, 48, 1, 1, 2, 0),     # three classes without a tap
-    (1, 20, 29, 31, 33, 7, 5, 3, 2),
-    (2, 16, 19, 40, 64, 3, 3, 4, 0),     # rows that no window reaches
+    (8, 128, 40, 36, 128, 3, 3, 1, 1, "conv2d_split 128x128 x2"),
+    (10, 160, 33, 31, 132, 5, 5, 1, 2, "conv2d_split 128x128 x2"),    # dy's channels padded to 144
+    (6, 128, 57, 55, 100, 3, 3, 2, 1, "conv2d_split 128x128 x2"),     # classes of different sizes
+    (24, 128, 57, 55, 72, 3, 3, 2, 1, "conv2d_split 128x128 x1"),
+    (8, 64, 57, 55, 100, 3, 3, 2, 1, "conv2d_split 64x128 x2"),
+    (16, 64, 57, 55, 100, 3, 3, 2, 1, "conv2d_split 64x128 x1"),
+    (12, 130, 41, 43, 72, 5, 5, 2, 2, "conv2d_split 128x128 x1"),     # two channels past a tile
+    (16, 96, 64, 64, 96, 1, 1, 2, 0, "conv2d_split 128x128 x1"),      # three classes without a tap
+    (12, 140, 59, 61, 70, 7, 5, 3, 2, "conv2d_split 128x128 x1"),     # stride 3, an oblong filter
+    (24, 64, 57, 60, 64, 3, 3, 4, 0, "conv2d_split 64x128 x1"),       # rows that no window reaches
+    (8, 64, 40, 36, 128, 3, 3, 1, 1, "conv2d_direct 64x64"),          # few pixels of the same
+    (2, 96, 33, 31, 48, 5, 5, 1, 2, "conv2d_small 32x32"),
+    (3, 40, 33, 30, 72, 3, 3, 2, 1, "conv2d_small 16x16"),
+    (2, 130, 20, 23, 37, 5, 5, 2, 2, "conv2d_small 16x16"),
+    (2, 24, 32, 32, 48, 1, 1, 2, 0, "conv2d_small 16x16"),
+    (1, 20, 29, 31, 33, 7, 5, 3, 2, "conv2d_small 16x16"),
+    (2, 16, 19, 40, 64, 3, 3, 4, 0, "conv2d_small 16x16"),
 ]
 
 
-@pytest.mark.parametrize("N,C_in,H,W,C_out,KH,KW,stride,pad", GRADIENT)
-def test_conv_split_bwd_input(dev, N, C_in, H, W, C_out, KH, KW, stride, pad):
+@pytest.mark.parametrize("N,C_in,H,W,C_out,KH,KW,stride,pad,kernel", GRADIENT)
+def test_conv_split_bwd_input(dev, N, C_in, H, W, C_out, KH, KW, stride, pad, kernel):
     case(f"conv split gradient {N} {C_in}->{C_out} {H}x{W} {KH}x{KW} stride {stride}")
     Ho, Wo = _out(H, KH, stride, pad), _out(W, KW, stride, pad)
     dy = prng.normal(6100, (N, C_out, Ho, Wo))
     w = prng.normal(6101, (C_out, C_in, KH, KW), std=float(np.sqrt(2.0 / (C_out * KH * KW))))
     got = _bwd_input(dev, dy, w, H, W, stride, pad)
+    assert _bwd_input.kernel == kernel
     x = torch.zeros(N, C_in, H, W, dtype=torch.float64, requires_grad=True)
     F.conv2d(x, torch.from_numpy(w).double(), None, stride, pad).backward(torch.from_numpy(dy).double())
     assert oracle.normwise_error(got, x.grad.numpy()) <= oracle.tolerance(C_out * KH * KW)
+    assert two_norm_error(got, x.grad.numpy()) <= fp32_sum_error(C_out * KH * KW)
 
 
 @pytest.mark.parametrize("stride", [1, 2])

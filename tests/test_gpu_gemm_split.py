@@ -3,6 +3,7 @@ edges of their tiles and k-steps, each operand layout, split K, and inputs at
 the ends of fp32's range, against fp64."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from lancius_amd import ACT_GELU, ACT_NONE, ACT_RELU, prng
@@ -87,6 +88,31 @@ def test_gemm_few_products_round_as_fp32(dev, K, layout):
     assert two_norm_error(got, A.astype(np.float64) @ B.astype(np.float64)) <= ROUNDING * np.sqrt((K + 1) / 2)
     if K == 1:
         assert np.array_equal(got, A * B)
+
+
+@pytest.mark.parametrize("layout", ["NN", "TN", "NT"])
+@pytest.mark.parametrize("M,K,N", [(3585, 64, 3590), (1537, 64, 2999), (1153, 288, 2304), (512, 4096, 512)])
+def test_gemm_split_keeps_its_low_products(dev, M, K, N, layout):
+    """Sums of x y - h yh - h ym - m yh (h, m: the first two bf16 parts of x and
+    y) leave what the parts' last products hl', mm', lh' add, 2^-17.8 rms: each of
+    them is 0.55 to 0.62 of a result.  Sums of terms of 1 round at 2^-25 a step,
+    2^-7 of what is left, and a tenth bounds that over the longest K here."""
+    case(f"gemm split low products {layout} {M}x{K}x{N}")
+
+    def parts(seed, shape):
+        x = torch.from_numpy(prng.normal(seed, shape))
+        h = x.bfloat16().float()
+        return tuple(t.numpy() for t in (x, h, (x - h).bfloat16().float()))
+
+    x, xh, xm = parts(81, (M, K // 4))
+    y, yh, ym = parts(82, (K // 4, N))
+    A = np.stack([x, -xh, -xh, -xm], -1).reshape(M, K)
+    B = np.stack([y, yh, ym, yh], 1).reshape(K, N)
+    ta, tb = layout[0] == "T", layout[1] == "T"
+    got = _run(dev, np.ascontiguousarray(A.T) if ta else A, np.ascontiguousarray(B.T) if tb else B, M, K, N, ta, tb)
+    assert any("gemm_f32_split" in k for k in _run.kernels)
+    err = two_norm_error(got, A.astype(np.float64) @ B.astype(np.float64))
+    assert err <= 0.1, err
 
 
 def test_gemm_split_k_is_repeatable(dev):

@@ -69,15 +69,18 @@ def test_soak_skinny_gemm(dev, M, K, N, act):
     dC.free()
 
 
-# Tile counts a little over a whole number per CU on a 256-CU part, so the
-# last tiles are shared (stream-K): 294 (128x64 tiles), 282 (64x64 tiles)
-# and the bench conv's 1568; a small grid split over all CUs (26 tiles, each
-# shared 4 ways).  5 / 5 / 2 / 3 inputs x 11 calls.
-CONV = [(6, 16, 56, 56, 128, 5), (23, 32, 28, 28, 64, 5), (32, 64, 56, 56, 128, 2), (1, 128, 28, 28, 256, 3)]
+# Tile counts a little over a whole number per CU on a 256-CU part, so the last
+# tiles are shared (stream-K): all of 294 (128x64) and 282 (64x64), the last of
+# 522 and 535; small grids split over all CUs (a tile shared up to 8 ways).  Two
+# more sizes that other kernels take: the bench conv and a single image.
+CONV = [(6, 16, 56, 56, 128, 5, "conv2d_direct 128x64 all shared"), (23, 32, 28, 28, 64, 5, "conv2d_direct 64x64 all shared"),
+        (5, 16, 37, 90, 144, 3, "conv2d_direct 128x64 tail shared"), (5, 16, 76, 90, 36, 3, "conv2d_direct 64x64 tail shared"),
+        (11, 352, 2, 24, 324, 3, "conv2d_direct 128x64 all shared"), (6, 304, 18, 22, 60, 3, "conv2d_direct 64x64 all shared"),
+        (32, 64, 56, 56, 128, 2, "conv2d_split 128x128 x1"), (1, 128, 28, 28, 256, 3, "conv2d_small 32x32")]
 
 
-@pytest.mark.parametrize("N,C_in,H,W,C_out,inputs", CONV)
-def test_soak_stream_k_conv(dev, N, C_in, H, W, C_out, inputs):
+@pytest.mark.parametrize("N,C_in,H,W,C_out,inputs,kernel", CONV)
+def test_soak_stream_k_conv(dev, N, C_in, H, W, C_out, inputs, kernel):
     n_out = N * C_out * H * W
     do = dev.alloc(n_out * 4)
     for s in range(inputs):
@@ -91,6 +94,7 @@ def test_soak_stream_k_conv(dev, N, C_in, H, W, C_out, inputs):
             case(f"soak stream-K conv N={N} C_in={C_in} {H}x{W} C_out={C_out} input {s} call {r}")
             dev.fill(do, float("nan"), n_out)
             dev.conv2d(do, dx, dw, db, N, C_in, H, W, C_out, 3, 3, 1, 1, act=ACT_RELU)
+            assert dev.launched()[0] == kernel
             got = dev.download(do, (N, C_out, H, W))
             if first is None:
                 first = got

@@ -6,8 +6,9 @@ decode kernel at every head-group width with and without float4 loads, the
 direct and implicit-GEMM convs with filters other than 3x3, the staged
 weight-gradient kernel, the unaligned small-batch MLP chains, the scalar
 tail of the elementwise kernels and the device-ceiling probes.  Each case
-names the variant it is there for; a kernel trace of the GPU suite lists
-every kernel of liblancius_hip.so as launched.  Tolerance as everywhere:
+names the variant it is there for; REACHED, REACHED_CONVS and REACHED_WGRADS
+compare the name with the kernel that ran, so a change of the dispatch that
+takes a case elsewhere fails here.  Tolerance as everywhere:
 1e-4 * max(1, sqrt(K)/32) with K the longest reduction."""
 import numpy as np
 import pytest
@@ -38,6 +39,7 @@ def _gemm_ex_case(dev, M, K, N, ta, tb, seed, act=ACT_GELU):
     dev.fill(dC, float("nan"), M * N)
     case(f"gemm_ex M={M} K={K} N={N} ta={ta} tb={tb} act={act}")
     dev.gemm_ex(dC, dA, dB, M, K, N, trans_a=ta, trans_b=tb, bias=db, act=act)
+    kernels = dev.launched(2)
     got = dev.download(dC, (M, N))
     for b in (dA, dB, db, dC):
         b.free()
@@ -46,8 +48,10 @@ def _gemm_ex_case(dev, M, K, N, ta, tb, seed, act=ACT_GELU):
     ref = oracle.matmul(A[rows], B) + bias.astype(np.float64)[None, :]
     ref = oracle.gelu(ref) if act == ACT_GELU else oracle.relu(ref) if act == ACT_RELU else ref
     assert oracle.normwise_error(got[rows], ref) <= oracle.tolerance(K)
+    return kernels[1] if kernels[0] == "splitk_reduce" else kernels[0]
 
 
+# sizes of the staged configurations' edges, whichever kernel takes them today
 # (M, K, N, ta, tb, variant)
 STAGED = [
     # 128x128/16 tiles (>= 256 of them) with transposed operands, float4 and scalar loads
@@ -77,6 +81,52 @@ STAGED = [
 @pytest.mark.parametrize("M,K,N,ta,tb,variant", STAGED, ids=[s[-1] for s in STAGED])
 def test_gemm_staged_variants(dev, M, K, N, ta, tb, variant):
     _gemm_ex_case(dev, M, K, N, ta, tb, seed=1300 + M + K + N)
+
+
+# (M, K, N, kernel): each fp32 kernel that the dispatch has left, at one of its
+# smallest sizes.  The kernels' names hold tile / k-tile x k-groups, the layout
+# (T: stored transposed) and the loads.
+REACHED = [
+    (34, 2268, 4, "gemm_f32_mfma 64x64/16 x1 NN float4 split K"),
+    (35, 2742, 1, "gemm_f32_mfma 64x64/16 x1 NN scalar split K"),
+    (2561, 2, 4652, "gemm_f32_mfma 128x128/16 x1 NN scalar"),
+    (10008, 4, 520, "gemm_f32_mfma 128x128/32 x2 NN float4"),
+    (10284, 3, 515, "gemm_f32_mfma 128x128/32 x2 NN scalar"),
+    (248, 2204, 984, "gemm_f32_mfma 128x128/32 x2 NN float4 split K"),
+    (5409, 3247, 129, "gemm_f32_mfma 128x128/32 x2 NN scalar split K"),
+    (264, 4, 10976, "gemm_f32_mfma 128x128/32 x4 NN float4"),
+    (10916, 5, 265, "gemm_f32_mfma 128x128/32 x4 NN scalar"),
+    (68, 4, 6088, "gemm_f32_mfma 64x64/64 x4 NN float4"),
+    (71, 1, 9045, "gemm_f32_mfma 64x64/64 x4 NN scalar"),
+    (384, 720, 988, "gemm_f32_mfma 64x64/64 x4 NN float4 split K"),
+    (833, 324, 897, "gemm_f32_mfma 64x64/64 x4 NN scalar split K"),
+    (948, 272, 1740, "gemm_f32_direct_kg x2"),
+    (641, 296, 1112, "gemm_f32_direct_kg x4"),
+    (67, 4, 7300, "gemm_f32_mfma 64x64/16 x1 NT float4"),
+    (11519, 1, 37, "gemm_f32_mfma 64x64/16 x1 NT scalar"),
+    (1, 2320, 1, "gemm_f32_mfma 64x64/16 x1 NT float4 split K"),
+    (1, 2221, 1, "gemm_f32_mfma 64x64/16 x1 NT scalar split K"),
+    (10912, 12, 272, "gemm_f32_mfma 128x128/16 x1 NT float4"),
+    (11284, 1, 276, "gemm_f32_mfma 128x128/16 x1 NT scalar"),
+    (68, 4, 8240, "gemm_f32_mfma 64x64/16 x1 TN float4"),
+    (33, 1, 11254, "gemm_f32_mfma 64x64/16 x1 TN scalar"),
+    (36, 2276, 4, "gemm_f32_mfma 64x64/16 x1 TN float4 split K"),
+    (33, 2618, 1, "gemm_f32_mfma 64x64/16 x1 TN scalar split K"),
+    (10912, 4, 260, "gemm_f32_mfma 128x128/16 x1 TN float4"),
+    (11530, 5, 261, "gemm_f32_mfma 128x128/16 x1 TN scalar"),
+    (68, 4, 7764, "gemm_f32_mfma 64x64/16 x1 TT float4"),
+    (11147, 1, 33, "gemm_f32_mfma 64x64/16 x1 TT scalar"),
+    (4, 2812, 2, "gemm_f32_mfma 64x64/16 x1 TT float4 split K"),
+    (1, 2320, 1, "gemm_f32_mfma 64x64/16 x1 TT scalar split K"),
+    (264, 16, 11568, "gemm_f32_mfma 128x128/16 x1 TT float4"),
+    (269, 12, 10940, "gemm_f32_mfma 128x128/16 x1 TT scalar"),
+]
+
+
+@pytest.mark.parametrize("M,K,N,kernel", REACHED, ids=[s[-1] for s in REACHED])
+def test_gemm_fp32_kernels_reached(dev, M, K, N, kernel):
+    layout = kernel.split(" ")[3] if "mfma" in kernel else "NN"
+    assert _gemm_ex_case(dev, M, K, N, layout[0] == "T", layout[1] == "T", seed=1350 + M + K + N) == kernel
 
 
 @pytest.mark.parametrize("M", [16, 32])
@@ -136,7 +186,8 @@ def test_decode_variants(dev, D, G):
     assert oracle.normwise_error(got, oracle.attention_decode(q, k, v, lens)) <= oracle.tolerance(Skv)
 
 
-# (N, C_in, H, W, C_out, K, stride, pad, variant)
+# (N, C_in, H, W, C_out, K, stride, pad, variant): sizes of the fp32 kernels'
+# edges, whichever kernel takes them today
 CONVS = [
     (2, 16, 20, 20, 128, 5, 1, 2, "direct 128x64 tiles, 5x5 filter"),
     (2, 16, 21, 19, 64, 1, 1, 0, "direct 64x64 tiles, 1x1 filter"),
@@ -171,9 +222,114 @@ def test_conv_variants(dev, N, C_in, H, W, C_out, K, stride, pad, variant):
     assert oracle.normwise_error(got, ref) <= oracle.tolerance(C_in * K * K)
 
 
+# (N, C_in, H, W, C_out, KH, KW, stride, pad, kernel): each fp32 kernel that the
+# dispatch has left, with 3x3 and other filters; C_in % 16 and C_out % 4 decide
+# between the direct kernel and the implicit GEMM
+REACHED_CONVS = [
+    (33, 16, 36, 9, 68, 3, 3, 1, 1, "conv2d_direct 128x64"),
+    (15, 16, 109, 1, 68, 7, 1, 1, 3, "conv2d_direct 128x64"),
+    (11, 352, 2, 24, 324, 3, 3, 1, 1, "conv2d_direct 128x64 all shared"),
+    (50, 272, 3, 1, 120, 7, 3, 1, 3, "conv2d_direct 128x64 all shared"),
+    (5, 16, 37, 90, 144, 3, 3, 1, 1, "conv2d_direct 128x64 tail shared"),
+    (36, 16, 46, 1, 272, 7, 1, 1, 3, "conv2d_direct 128x64 tail shared"),
+    (45, 16, 33, 7, 36, 3, 3, 1, 1, "conv2d_direct 64x64"),
+    (47, 16, 83, 1, 44, 5, 3, 1, 2, "conv2d_direct 64x64"),
+    (6, 304, 18, 22, 60, 3, 3, 1, 1, "conv2d_direct 64x64 all shared"),
+    (1, 304, 4, 39, 52, 7, 7, 1, 3, "conv2d_direct 64x64 all shared"),
+    (5, 16, 76, 90, 36, 3, 3, 1, 1, "conv2d_direct 64x64 tail shared"),
+    (41, 144, 121, 1, 52, 7, 1, 1, 3, "conv2d_direct 64x64 tail shared"),
+    (1, 1, 1, 1, 67, 3, 3, 1, 1, "conv2d_implicit_gemm 128x64"),
+    (1, 3, 1, 1, 73, 4, 3, 1, 2, "conv2d_implicit_gemm 128x64"),
+    (1, 2, 1, 1, 33, 3, 3, 1, 1, "conv2d_implicit_gemm 64x64"),
+    (1, 1, 1, 1, 34, 4, 4, 1, 2, "conv2d_implicit_gemm 64x64"),
+    (1, 1, 1, 1, 1, 3, 3, 1, 1, "conv2d_implicit_gemm 32x128"),
+    (1, 1, 1, 1, 1, 1, 1, 3, 0, "conv2d_implicit_gemm 32x128"),
+    (7, 16, 83, 53, 4, 3, 3, 1, 1, "conv2d_implicit_gemm 32x128 per channel"),
+    (57, 16, 127, 1, 4, 4, 1, 1, 2, "conv2d_implicit_gemm 32x128 per channel"),
+]
+
+
+@pytest.mark.parametrize("N,C_in,H,W,C_out,KH,KW,stride,pad,kernel", REACHED_CONVS)
+def test_conv_fp32_kernels_reached(dev, N, C_in, H, W, C_out, KH, KW, stride, pad, kernel):
+    x = prng.normal(1750 + C_in, (N, C_in, H, W))
+    w = prng.normal(1751 + C_out, (C_out, C_in, KH, KW), 0, float(np.sqrt(2.0 / (C_in * KH * KW))))
+    bias = prng.normal(1752, (C_out,), 0, 0.1)
+    Ho, Wo = (H + 2 * pad - KH) // stride + 1, (W + 2 * pad - KW) // stride + 1
+    dx, dw, db, do = _up(dev, x), _up(dev, w), _up(dev, bias), dev.alloc(4 * N * C_out * Ho * Wo)
+    dev.fill(do, float("nan"), N * C_out * Ho * Wo)
+    case(f"conv {kernel} {N} {C_in}->{C_out} {H}x{W} {KH}x{KW}")
+    dev.conv2d(do, dx, dw, db, N, C_in, H, W, C_out, KH, KW, stride, pad, act=ACT_RELU)
+    ran = dev.launched()[0]
+    got = dev.download(do, (N, C_out, Ho, Wo))
+    for t in (dx, dw, db, do):
+        t.free()
+    ref = oracle.relu(oracle.conv2d(x, w, stride, pad, False) + bias.astype(np.float64)[None, :, None, None])
+    assert ran == kernel
+    assert oracle.normwise_error(got, ref) <= oracle.tolerance(C_in * KH * KW)
+
+
+# gradients by the input of the same kernels: (N, channels of dy, H, W, channels of dx, K)
+REACHED_GRADIENTS = [
+    (16, 16, 6, 113, 68, 3, "conv2d_direct 128x64"),
+    (1, 352, 13, 41, 356, 3, "conv2d_direct 128x64 all shared"),
+    (15, 16, 74, 15, 136, 3, "conv2d_direct 128x64 tail shared"),
+    (7, 16, 77, 19, 36, 3, "conv2d_direct 64x64"),
+    (8, 288, 7, 50, 36, 3, "conv2d_direct 64x64 all shared"),
+    (49, 16, 113, 6, 36, 3, "conv2d_direct 64x64 tail shared"),
+    (1, 1, 43, 65, 97, 3, "conv2d_implicit_gemm 128x64"),
+    (9, 1, 85, 8, 33, 3, "conv2d_implicit_gemm 64x64"),
+    (33, 1, 3, 23, 53, 7, "conv2d_implicit_gemm 64x64"),
+    (18, 1, 65, 12, 1, 3, "conv2d_implicit_gemm 32x128"),
+    (36, 16, 122, 7, 4, 3, "conv2d_implicit_gemm 32x128 per channel"),
+]
+
+
+@pytest.mark.parametrize("N,Co,H,W,Ci,K,kernel", REACHED_GRADIENTS)
+def test_conv_gradient_fp32_kernels_reached(dev, N, Co, H, W, Ci, K, kernel):
+    g, w = prng.normal(1770 + Co, (N, Co, H, W)), prng.normal(1771 + Ci, (Co, Ci, K, K), 0, float(np.sqrt(2.0 / (Co * K * K))))
+    dg, dw, do = _up(dev, g), _up(dev, w), dev.alloc(4 * N * Ci * H * W)
+    dev.fill(do, float("nan"), N * Ci * H * W)
+    case(f"conv gradient {kernel} {N} {Co}->{Ci} {H}x{W} {K}x{K}")
+    dev.conv2d_bwd_input(do, dg, dw, N, Ci, H, W, Co, H, W, K, K, 1, K // 2)
+    ran = dev.launched()[0]
+    got = dev.download(do, (N, Ci, H, W))
+    for t in (dg, dw, do):
+        t.free()
+    ref = oracle.conv2d_bwd_input(g.astype(np.float32), w.astype(np.float32), (N, Ci, H, W), 1, K // 2)
+    assert ran == kernel
+    assert oracle.normwise_error(got, ref) <= oracle.tolerance(Co * K * K)
+
+
+# (N, C_in, H, W, C_out, K, stride, pad, kernel)
+REACHED_WGRADS = [
+    (6, 1, 27, 1, 124, 1, 2, 0, "conv2d_wgrad_mfma"),
+    (10, 5, 8, 1, 2, 5, 2, 2, "conv2d_wgrad_mfma"),
+    (1, 4, 10, 4, 125, 1, 1, 0, "conv2d_wgrad_direct"),
+    (5, 2, 16, 1, 5, 5, 1, 2, "conv2d_wgrad_direct"),
+    (3, 80, 64, 50, 144, 3, 3, 0, "conv2d_wgrad_direct"),
+]
+
+
+@pytest.mark.parametrize("N,Ci,H,W,Co,K,stride,pad,kernel", REACHED_WGRADS)
+def test_wgrad_fp32_kernels_reached(dev, N, Ci, H, W, Co, K, stride, pad, kernel):
+    Ho, Wo = (H + 2 * pad - K) // stride + 1, (W + 2 * pad - K) // stride + 1
+    x, g = prng.normal(1780 + Ci, (N, Ci, H, W)), prng.normal(1781 + Co, (N, Co, Ho, Wo))
+    dx, dg, do = _up(dev, x), _up(dev, g), dev.alloc(4 * Co * Ci * K * K)
+    case(f"wgrad {kernel} {N} {Ci}->{Co} {H}x{W} {K}x{K} stride {stride}")
+    dev.conv2d_bwd_weight(do, dg, dx, N, Ci, H, W, Co, Ho, Wo, K, K, stride, pad)
+    ran = dev.launched(2)
+    got = dev.download(do, (Co, Ci, K, K))
+    for t in (dx, dg, do):
+        t.free()
+    ref = oracle.conv2d_bwd_weight(g.astype(np.float32), x.astype(np.float32), (Co, Ci, K, K), stride, pad)
+    assert kernel in ran
+    assert oracle.normwise_error(got, ref) <= oracle.tolerance(N * Ho * Wo)
+
+
 def test_conv_wgrad_staged_128(dev):
     """Weight gradient with more than 64 output channels and H_out * W_out
-    not a multiple of 4: the register-staged kernel at 128 x 64 tiles."""
+    not a multiple of 4: the register-staged kernel's 128 x 64 tiles (or the
+    split products)."""
     N, Ci, H, W, Co = 2, 8, 7, 7, 96
     x, g = prng.normal(1800, (N, Ci, H, W)), prng.normal(1801, (N, Co, H, W))
     dx_, dg_, dw_ = _up(dev, x), _up(dev, g), dev.alloc(4 * Co * Ci * 9)
