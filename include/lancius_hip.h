@@ -72,6 +72,13 @@ LANCIUS_HIP_EXPORT int lancius_hip_timer_stop(lancius_hip_ctx* ctx, float* elaps
 
 /* ---- kernels (device pointers, fp32, row-major) --------------------- */
 
+/* Large products, convolutions, their gradients and attention run on the bf16
+ * matrix cores with each fp32 operand in three bf16 parts: errors as of fp32
+ * sums or smaller, over all of fp32's range.  Tiles that meet an infinity, a
+ * NaN, an operand of 2^112 or more or a sum of 2^96 or more are computed a
+ * second time with the fp32 instructions: the values are those of fp32
+ * arithmetic, and a call whose every tile does takes up to 3.7 times as long. */
+
 /* C[M,N] = epilogue(A[M,K] . B[K,N]).
  * Epilogue order: y = acc + bias[n] (bias may be NULL); y = act(y) with act
  * any LANCIUS_HIP_ACT_*; y = y + residual[m,n] (residual may be NULL; it
@@ -88,7 +95,9 @@ LANCIUS_HIP_EXPORT int lancius_hip_gemm_f32(lancius_hip_ctx* ctx, float* C, cons
  * fixed scratch array of LANCIUS_HIP_NOALLOC_SCRATCH_BYTES inside the
  * library, one per GPU, held until the process ends; it never grows the
  * context workspace and calls no hipMalloc or hipFree.  Same kernels and same
- * split choice as lancius_hip_gemm_f32, hence the same bits.  A shape whose
+ * split choice as lancius_hip_gemm_f32, hence the same bits (recorded into a
+ * graph, lancius_hip_gemm_f32 has them only on a context that has the scratch
+ * memory: see lancius_hip_capture_begin).  A shape whose
  * partial sums would exceed the scratch returns -3 before anything is
  * launched.  Every call on one GPU shares that GPU's scratch: calls that
  * overlap on one GPU (two streams or two host threads) race, so order them. */

@@ -1200,7 +1200,8 @@ constexpr int kBK = 16;
 constexpr size_t kMaxSplitBytes = (size_t)256 << 20;
 
 // Which kernel a product takes when it is too large for the skinny one, from
-// what each costs on this chip (us, one launch alone, 256 CUs):
+// what each costs on this chip (us, one launch alone, 256 CUs; on a partition
+// of fewer the choice is only less apt):
 //  * split-product tiles (gemm_f32_split): a round of one tile per CU costs a
 //    start and a time per unit of K.  Measured at 4096 x 4096 x K (256 x 256:
 //    one round) and 2048 x 2048 x 2048 (128 x 128: one round):
@@ -1262,6 +1263,9 @@ GemmPlan gemm_plan(size_t count, size_t M, size_t K, size_t N, bool plain, bool 
 
 // The skinny kernel's time in us: a launch, then what one workgroup takes for
 // its K slice and the adding of slices; scalar rows of B (N % 4) slow it down.
+// Up to 16 rows (8 and 16 measured): one slice 4.6 to 5.3; more, up to 64 columns
+// and K <= 1664 5.6 to 6.4 (its lower end is taken: small tiles take 4.2 to 6.0
+// there and gemm_small_plan says up to 6.8); others 5.9 to 6.8.
 double skinny_us(size_t count, size_t M, size_t K, size_t N, bool vb) {
     const double k = (double)K, bytes = 4.0 * (double)count * k * N;
     const double us = vb ? (M <= 16 ? (K <= 512 ? 4.9 : K <= 1664 && N <= 64 ? 5.8 : 6.3) : (K <= 512 ? 7.0 : 8.7))
@@ -1394,15 +1398,20 @@ int gemm_dispatch(lancius_hip_ctx* ctx, size_t count, float* const* C, const flo
 
     // Configurations (BM x BN / BK, k-groups): 2 = 64x64/16, 6 = 128x128/16
     // built for 4 workgroups per CU, 7 = 128x128/32 x2, 8 = 128x128/32 x4,
-    // 9 = 64x64/64 x4.  Chosen by the number of 128x128 tiles (one per CU
-    // fills the chip once), measured on MI355X:
-    //  * >= 768: 6 (operands beyond 32-bit offsets, K < 3);
+    // 9 = 64x64/64 x4.  They are left with what the kernels above do not
+    // take or are estimated slower at: a K of a few dozen, long K's of small
+    // grids, unaligned operands, both operands transposed, operands beyond
+    // 32-bit offsets, a capture without scratch memory.  Chosen by the number
+    // of 128x128 tiles (one per CU fills the chip once; the lines were
+    // measured when these kernels took larger products too):
+    //  * >= 768: 6 (plain operands: beyond 32-bit offsets, K < 3);
     //  * 384 .. 767: 7 (two 8-wave workgroups per CU);
-    //  * 256 .. 383: 8, 16 waves on the CU's one tile (4096x1024x1024: 110 ->
-    //    103 us);
-    //  * fewer, K >= 2048: 7 with split-K (1024x4096x1024: 137 -> 103 us);
-    //  * fewer, shorter K: 9 (1024^3: 38.9 -> 34.0 us), or 2 for small
-    //    grids and transposed operands.
+    //  * 256 .. 383: 8, 16 waves on the CU's one tile (against 7 at
+    //    4096x1024x1024 110 -> 103 us);
+    //  * fewer, K >= 2048: 7 with split-K (against one K range at
+    //    1024x4096x1024 137 -> 103 us);
+    //  * fewer, shorter K: 9 (against 2 at 1024^3 38.9 -> 34.0 us), or 2 for
+    //    small grids and transposed operands.
     // Split-K when the grid still leaves CUs idle and K is long enough:
     // enough K ranges for ~512 workgroups, each >= 128 deep.
     const size_t t64 = count * ((M + 63) / 64) * ((N + 63) / 64);
