@@ -24,9 +24,10 @@ constexpr float kQueryUp = 0x1p32f;
 // blocks of the same queries (grids of at most one tile per CU).
 //
 // What bounds it: at D = 64 the matrix cores' 48 products a step and the 230
-// vector instructions of the softmax, the splits of P and of the staged keys,
-// half the matrix-core time each (MFMA busy 0.49, vector issue 0.48 at B8 H16
-// S=2048 before the two were overlapped); at D = 128 the products.
+// vector instructions of the softmax, the splits of P and of the staged keys
+// (B8 H16 S=2048 causal: matrix cores busy 0.52, vector unit 0.56 of the busy
+// CUs' cycles); at D = 128 the products that wait for the softmax (busy 0.57,
+// vector unit 0.45 in a ragged causal prefill).
 //  * S^T = K Q^T and O^T += V^T P^T with v_mfma_f32_32x32x16_bf16: a lane owns
 //    one query in both, and its 16 scores, in register order, are the two P^T
 //    operands of the block: keys 16 s + 8 (e / 4) + 4 half + e % 4 for element

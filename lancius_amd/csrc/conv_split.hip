@@ -14,8 +14,8 @@
 // that miss (at stride 2 a quarter of the products of one convolution over
 // the spread-out dy).
 //
-// Measured, fp32 kernels -> this: N32 64->128 3x3 56^2 131 -> 99 us forward,
-// 142 -> 123 its gradient; N32 128->128 28^2 86 -> 49; the gradient at stride 2
+// Measured, fp32 kernels -> this: N32 64->128 3x3 56^2 131 -> 100 us forward,
+// 142 -> 129 its gradient; N32 128->128 28^2 86 -> 49; the gradient at stride 2
 // of N16 64->128 56^2 3263 (one thread an element) -> 32.  What bounds the
 // first: 784 tiles on 512 slots, a second round half full; sharing the last
 // tiles by k-steps through the point of coherence cost more than it saved (99

@@ -11,8 +11,8 @@
 // gradients wgrad_reduce (conv.hip) adds in order.
 //
 // N32 64->128 3x3 56^2 (5 tiles of 128 x 128, 51 ranges of 123 steps): fp32
-// kernel 143 us, this 97 (1.53 us a pair of steps, of which the products are
-// 0.75; X's addresses, masks and splits fill the rest); N32 256->256 14^2 87 -> 58.
+// kernel 143 us, this 98 (matrix cores busy 0.51 of the busy CUs' cycles, the
+// vector unit 0.54: X's addresses, masks and splits); N32 256->256 14^2 87 -> 58.
 #include <algorithm>
 
 #include "conv.hpp"
