@@ -165,7 +165,7 @@ def test_cross_entropy_golden(dev):
         b.free()
 
 
-@pytest.mark.parametrize("R,Cc", [(1, 2), (64, 10), (1000, 1000), (8192, 10)])
+@pytest.mark.parametrize("R,Cc", [(1, 2), (64, 10), (1000, 1000), (8192, 10), (1, 677), (3, 300), (16, 257), (17, 300), (5, 16), (65, 16), (3, 65)])
 def test_cross_entropy(dev, R, Cc):
     x = prng.normal(700 + R, (R, Cc), std=3.0)
     lab = (prng.uniform(701 + R, (R,), 0, 1) * Cc).astype(np.int64) % Cc
