@@ -1270,14 +1270,21 @@ int launch_tile(lancius_hip_ctx* ctx, ConvParams& p, int tile) {
 // tiles, three workgroups a CU and at least 256 pixels each, then the sum of
 // the splits.  Fitted with wgrad_split_plan's to 90 shapes: N32 64->128 56^2
 // 144 (split products 103), N32 256->256 14^2 87 (58), N2 64->64 56^2 17 (17),
-// N5 112->160 1x1 at stride 2 of 11x8 10 (16).
+// N5 112->160 1x1 at stride 2 of 11x8 10 (16).  Against the estimates of one short
+// range that were the same as of long ones, 44 of 520 random gradients had gone
+// to split products that the fp32 kernels do faster (N13 16->4 1x1 of 2x1 pixels
+// 11.3 us, 4.3 here); now three, by 15% at most.
 double wgrad_fp32_us(size_t C_out, size_t J, size_t P, bool direct) {
     const double wide = C_out > 64 ? 1.0 : 0.62;
     const double tiles = std::ceil(C_out / (C_out > 64 ? 128.0 : 64.0)) * std::ceil(J / 64.0);
     const double splits = std::max(1.0, std::min(std::floor(768.0 / tiles), std::floor(P / 256.0)));
     const double kt = std::ceil(P / splits / 16.0);
     const double us = 4.5 + 0.58 * wide * kt * std::max(0.55, tiles * splits / 256) + (splits > 1 ? 6.5 : 0.0);
-    return direct ? us : 5.0 + 1.6 * us;  // images of a pixel count that is no multiple of 4: the staged kernel
+    // images of a pixel count that is no multiple of 4: the staged kernel.  One
+    // range of few pixels costs it a step of 32 each (up to 32 pixels 4.3 to 5.3
+    // us, more than 64 channels 5.8 to 7; 80 8.8, 12; 300 21.4, 30).
+    if (!direct && P < 512 && tiles <= 768) return C_out > 64 ? 4.0 + 2.65 * std::ceil(P / 32.0) : 3.5 + 1.8 * std::ceil(P / 32.0);
+    return direct ? us : 5.0 + 1.6 * us;
 }
 
 }  // namespace
@@ -1454,7 +1461,7 @@ extern "C" int lancius_hip_conv2d_bwd_weight_f32(lancius_hip_ctx* ctx, float* dw
         double us = 0.0;
         wgrad_split_plan(sp, (size_t)cu_count(ctx), &us);
         if (workspace_ready(ctx, sp.splits > 1 ? (size_t)sp.splits * C_out * J * sizeof(float) : 0) &&
-            us < 1.15 * wgrad_fp32_us(C_out, J, N * H_out * W_out, H_out * W_out % 4 == 0 && H_out * W_out >= 16)) {
+            us < (wgrad_split_few(sp) ? 1.0 : 1.15) * wgrad_fp32_us(C_out, J, N * H_out * W_out, H_out * W_out % 4 == 0 && H_out * W_out >= 16)) {
             if (sp.splits > 1) {
                 void* ws = nullptr;
                 if (int rc = workspace(ctx, (size_t)sp.splits * C_out * J * sizeof(float), &ws)) return rc;

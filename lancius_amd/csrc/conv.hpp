@@ -48,6 +48,7 @@ struct WgradSplitParams {
 bool wgrad_split_fits(const WgradSplitParams& p);
 // Sets chunk and splits for a grid of about one workgroup per CU; us: an estimate of the launch.
 void wgrad_split_plan(WgradSplitParams& p, size_t cus, double* us);
+bool wgrad_split_few(const WgradSplitParams& p);  // one range of few pixels
 int launch_wgrad_split(lancius_hip_ctx* ctx, WgradSplitParams& p);
 
 }  // namespace lancius

@@ -269,6 +269,8 @@ bool wgrad_split_fits(const WgradSplitParams& p) {
            (size_t)p.Ho * p.stride < ((size_t)1 << 30);
 }
 
+bool wgrad_split_few(const WgradSplitParams& p) { return p.splits == 1 && p.chunk <= 32; }
+
 void wgrad_split_plan(WgradSplitParams& p, size_t cus, double* us) {
     p.row_oct = (p.Wo + 7) / 8;
     p.octets = p.N * p.Ho * p.row_oct;
@@ -285,6 +287,8 @@ void wgrad_split_plan(WgradSplitParams& p, size_t cus, double* us) {
     const double rounds = (double)((tiles * p.splits + cus - 1) / cus);
     const double parts = p.splits > 1 ? 3.0 + 4.0 * p.C_out * p.J * p.splits * 2.0 / 4e6 : 0.0;
     *us = rounds * (8.0 + (bm == 128 ? 0.68 : 0.4) * p.chunk) + parts;
+    // one short range: two steps 5.4 us (7.0), sixteen 12.4 (16.5), thirty 20
+    if (wgrad_split_few(p) && rounds == 1.0) *us = bm == 128 ? 5.6 + 0.69 * p.chunk : 4.4 + 0.5 * p.chunk;
 }
 
 int launch_wgrad_split(lancius_hip_ctx* ctx, WgradSplitParams& p) {

@@ -307,6 +307,14 @@ REACHED_WGRADS = [
     (1, 4, 10, 4, 125, 1, 1, 0, "conv2d_wgrad_direct"),
     (5, 2, 16, 1, 5, 5, 1, 2, "conv2d_wgrad_direct"),
     (3, 80, 64, 50, 144, 3, 3, 0, "conv2d_wgrad_direct"),
+    # few pixels: one short range, either kernel
+    (13, 16, 4, 2, 4, 1, 2, 0, "conv2d_wgrad_mfma"),
+    (7, 23, 4, 1, 25, 1, 3, 0, "conv2d_wgrad_mfma"),
+    (10, 16, 4, 3, 64, 1, 2, 0, "conv2d_wgrad_mfma"),
+    (17, 16, 7, 13, 4, 7, 3, 0, "conv2d_wgrad_mfma"),
+    (2, 32, 3, 4, 132, 1, 1, 0, "conv2d_wgrad_mfma"),
+    (3, 16, 9, 13, 12, 3, 1, 1, "wgrad_split 64x128"),
+    (2, 16, 9, 13, 130, 3, 1, 1, "wgrad_split 128x128"),
 ]
 
 
