@@ -1233,6 +1233,23 @@ bool use_split(lancius_hip_ctx* ctx, const ConvParams& q, ConvSplitParams* sp) {
     return split < fp32 && (size_t)q.Kdim >= kSplitLeast;
 }
 
+// Whether a gradient whose elements see few products each (or that the split
+// products leave to the fp32 instructions) is better a thread an element: 0.2
+// us a tap and channel in a chain, 0.88 us a million of them, against `us` of
+// the tiles, their filter's layout, and the stores of the stride's classes,
+// each into every s-th value of the same lines.  N2 4->16 3x3 stride 3 of 78x105
+// 12.2 us here, 16.9 as tiles; N22 of 12x65 14.2, 17.6; N8 4->22 of 90x43 29, 18.
+bool dgrad_direct_ahead(const ConvSplitParams& p, double us, int tile) {
+    const size_t s = (size_t)p.stride;
+    const size_t seen = (size_t)p.C_in * ((p.KH + s - 1) / s) * ((p.KW + s - 1) / s);
+    if (seen > 8 && p.C_in >= (int)kSplitLeast) return false;
+    const double products = (double)p.C_in * p.KH * p.KW, elements = (double)p.N * p.C_out * p.Ho * p.Wo;
+    const double direct = 4.0 + std::max(0.2 * products, 0.88e-6 * elements * products);
+    const double pixels = (double)p.N * (double)((p.Ho + s - 1) / s) * (double)((p.Wo + s - 1) / s);
+    const double tiles = (double)(s * s) * std::ceil((double)p.C_out / tile) * std::ceil(pixels / tile);
+    return direct < us + (s <= 2 ? 2.2 : 4.2) + 3e-3 * (double)(s - 1) * tiles;
+}
+
 // One launch per run of images whose input stays under 2 GiB (the direct
 // kernel's 32-bit input offsets); the images of a conv are independent, so
 // the split changes no result.  p describes the whole batch.
@@ -1400,16 +1417,19 @@ extern "C" int lancius_hip_conv2d_bwd_input_f32(lancius_hip_ctx* ctx, float* dx,
     if (!as_conv) {
         ConvSplitParams sp{dx, dy, nullptr, nullptr, (int)N, (int)C_out, (int)((C_out + 15) / 16 * 16), (int)H_out, (int)W_out,
                            (int)C_in, (int)K_h, (int)K_w, (int)stride, (int)pad, (int)H, (int)W, 1, LANCIUS_HIP_ACT_NONE, 0, 0};
-        // (up to a dozen products an element, or sizes beyond its offsets, the
+        // (filters of up to a dozen products, or sizes beyond its offsets, the
         // split-product kernel leaves to the direct one: N15 4->8 1x1 107x11
         // 6.1 us against 8.6; N16 64->128 3x3 56^2 the other way, 3263
         // against 32)
         if (C_out * K_h * K_w > 12 && stride <= 16 && K_h < (1u << 15) && K_w < (1u << 15) && C_out > 0 && pad < (1u << 30) && conv_split_fits(sp) &&
             workspace_ready(ctx, conv_split_weight_bytes(sp))) {
             int tile;
-            if (conv_small_plan(sp, &tile) < conv_split_us(sp) || C_out < kSplitLeast) sp.small_tile = tile;
-            const int rc = launch_conv_split(ctx, sp, w);
-            return rc ? rc : ok();
+            const double small = conv_small_plan(sp, &tile), split = conv_split_us(sp);
+            if (small < split || C_out < kSplitLeast) sp.small_tile = tile;
+            if (!dgrad_direct_ahead(sp, sp.small_tile ? small : split, tile)) {
+                const int rc = launch_conv_split(ctx, sp, w);
+                return rc ? rc : ok();
+            }
         }
         const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>((total + 255) / 256, 16384));
         hipLaunchKernelGGL(dgrad_direct, dim3(grid), dim3(256), 0, ctx->stream, dx, dy, w, (int)N, (int)C_in, (int)H,

@@ -106,6 +106,10 @@ GRADIENT = [
     (24, 64, 57, 60, 64, 3, 3, 4, 0, "conv2d_split 64x128 x1"),       # rows that no window reaches
     (8, 64, 40, 36, 128, 3, 3, 1, 1, "conv2d_direct 64x64"),          # few pixels of the same
     (2, 96, 33, 31, 48, 5, 5, 1, 2, "conv2d_small 32x32"),
+    (2, 16, 78, 105, 4, 3, 3, 3, 0, "conv2d_dgrad_direct"),           # one tap of four channels an element
+    (22, 16, 12, 65, 4, 3, 3, 3, 1, "conv2d_dgrad_direct"),
+    (20, 2, 81, 107, 2, 7, 7, 2, 3, "conv2d_dgrad_direct"),           # two channels: no split products
+    (8, 22, 90, 43, 4, 3, 3, 3, 1, "conv2d_small 32x32"),             # more pixels of the first
     (3, 40, 33, 30, 72, 3, 3, 2, 1, "conv2d_small 16x16"),
     (2, 130, 20, 23, 37, 5, 5, 2, 2, "conv2d_small 16x16"),
     (2, 24, 32, 32, 48, 1, 1, 2, 0, "conv2d_small 16x16"),
